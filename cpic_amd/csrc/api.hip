@@ -160,10 +160,10 @@ dev_free(cpic_dev *d)
 	hipFree(d->E); hipFree(d->costab); hipFree(d->tw);
 	cpic_parts_free(d, 0);
 	cpic_parts_free(d, 1);
-	hipFree(d->bk.start); hipFree(d->bk.cap); hipFree(d->bk.n1); hipFree(d->bk.res);
-	hipFree(d->bk.n2);
+	hipFree(d->bk.start); hipFree(d->bk.cap); hipFree(d->bk.base); hipFree(d->bk.cnt);
 	hipFree(d->order);
-	hipFree(d->border);
+	hipFree(d->units);
+	hipFree(d->holes);
 	hipFree(d->dpart);
 	hipFree(d->lv.x); hipFree(d->lv.y); hipFree(d->lv.ux); hipFree(d->lv.uy);
 	hipFree(d->lv.id); hipFree(d->lv.Ex); hipFree(d->lv.Ey); hipFree(d->lv.dst);
@@ -420,6 +420,7 @@ batch_create(const cpic_dev_desc_t *descs, int P, cpic_dev_t **out)
 	d->ghat_n = ghat;
 	d->ntiles = (int) tiles;
 	d->nb = (int) buckets;
+	d->bk.nb = d->nb;
 	d->rowblocks = (int) rows;
 	d->colblocks = (int) cols;
 	d->nodeblocks = (int) nblk;
@@ -449,14 +450,12 @@ batch_create(const cpic_dev_desc_t *descs, int P, cpic_dev_t **out)
 			(ret = alloc_zero((void **) &d->geo, sizeof(Geo) * P)) ||
 			(ret = alloc_zero((void **) &d->pre, sizeof(int) * PRE_COUNT * (P + 1))) ||
 			(ret = alloc_zero((void **) &d->order, sizeof(int) * d->ntiles)) ||
-			(ret = alloc_zero((void **) &d->border, sizeof(int) * d->nb)) ||
 			(ret = alloc_zero((void **) &d->dpart,
 					sizeof(double) * (DIAG_SPREAD * DIAG_LINE * (size_t) P + DIAG_LINE))) ||
 			(ret = alloc_zero((void **) &d->bk.start, sizeof(int64_t) * d->nb)) ||
 			(ret = alloc_zero((void **) &d->bk.cap, sizeof(int32_t) * d->nb)) ||
-			(ret = alloc_zero((void **) &d->bk.n1, sizeof(int32_t) * d->nb)) ||
-			(ret = alloc_zero((void **) &d->bk.res, sizeof(int32_t) * d->nb)) ||
-			(ret = alloc_zero((void **) &d->bk.n2, sizeof(int32_t) * d->nb)) ||
+			(ret = alloc_zero((void **) &d->bk.base, sizeof(BucketBase) * 2 * d->nb)) ||
+			(ret = alloc_zero((void **) &d->bk.cnt, sizeof(BucketCnt) * 2 * d->nb)) ||
 			(ret = alloc_zero((void **) &d->lv.count, sizeof(int32_t) * 2)) ||
 			(ret = cpic_fft_init(d)) ||
 			(ret = cpic_parts_init(d)))

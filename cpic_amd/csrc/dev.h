@@ -15,12 +15,19 @@
 //            E (double2 or float2 (Ex,Ey) pairs).
 //   particles buckets, one per (plasma, tile, species), tile-major inside a
 //            plasma; state x, y, ux, uy in groups of 64 slots (+ optional id,
-//            Ex, Ey arrays).  A bucket
-//            owns slots [start, start+cap): segment 1 holds n1 particles at
-//            [0, n1), segment 2 holds n2 fallback particles at
-//            [cap-res, cap-res+n2), where res is the number of particles that
-//            left the bucket in the last push (their slots are kept free so a
-//            leaver whose destination is full can always return).
+//            Ex, Ey arrays).  A bucket owns slots [start, start+cap).  Two ways
+//            to keep them (push_in_place()):
+//            in place (up to some size of the whole state): slots [0, n) are in
+//            use.  A particle keeps its slot while it stays in the tile; the
+//            slot of one that left becomes a hole (x = NaN) and waits in the
+//            bucket's ring of holes, from which arriving particles take their
+//            slots before the bucket grows.  The holes a push makes can be
+//            taken from the next step on: until then they stay free for
+//            leavers that find their destination full;
+//            compact (larger states): each push packs the particles that stay
+//            at the front of the same bucket of another buffer.  Arriving
+//            particles follow; the last `out` slots, as many as left, stay
+//            free for leavers that find their destination full.
 //   FP64 mode stores absolute positions (the reference's r); FP32 mode
 //   stores positions in cell units relative to the bucket tile's origin.
 #pragma once
@@ -71,12 +78,20 @@ struct Geo {
 // Work-list prefix arrays (P+1 entries each), concatenated.
 enum { PRE_TILE = 0, PRE_ROW, PRE_COL, PRE_NODEBLK, PRE_BUCKET, PRE_COUNT };
 
+// Metadata of the buckets.  What a step leaves for its arrivals (base) and what
+// the step counts (cnt) alternate between two arrays of nb entries each,
+// index (step parity) * nb + bucket: the push of parity p reads both of
+// parity 1-p, writes base[p] and counts into cnt[p], which k_append of parity
+// p also counts into; bucket_now() gives the state after a step.
+struct BucketBase { int32_t n, head, holes, pad; };  // slots in use; ring: first hole, holes
+struct BucketCnt { int32_t in, out, back, pad; };    // arrived, left, returned to their source
 struct Buckets {
 	int64_t *start;
 	int32_t *cap;
-	int32_t *n1;
-	int32_t *res;
-	int32_t *n2;
+	BucketBase *base;        // [2][nb]
+	BucketCnt *cnt;          // [2][nb]
+	int nb;
+	int compact;             // kept compact, not in place
 };
 
 // Particle state (double or float) in groups of PGROUP particles: group k
@@ -155,6 +170,7 @@ struct cpic_dev {
 	int rowblocks, colblocks, nodeblocks;
 	int fft_nt_row, fft_nt_col;   // threads per block of the FFT row and column passes
 	size_t lds_push, lds_rows, lds_cols;
+	int phi_apart;           // the push's potential region has LDS of its own
 
 	// fields
 	double *rho[2];
@@ -171,12 +187,17 @@ struct cpic_dev {
 	int lgN;
 
 	// particles
-	Parts p[2];              // [cur] in use, [1-cur] spare for rebuilds
+	Parts p[2];              // [cur] in use, [1-cur] the compacting push's other buffer
+	                         // and the target of the next re-sort
 	int pcur;
 	int64_t pcap[2];
+	int32_t *holes;          // [holecap]: bucket b's ring of holes at [start, start+cap)
+	int64_t holecap;
 	Buckets bk;
 	int *order;              // [ntiles] tile taken by each block of the tile kernels
-	int *border;             // [nb] bucket taken by each block of the push
+	int2 *units;             // [nunits] the push's work: (bucket, part | parts << 16)
+	int nunits;
+	int unitcap;
 	double *dpart;           // [P][DIAG_SPREAD][DIAG_LINE]: the push's kinetic, px, py sums,
 	                         // then one line whose first 8 bytes hold their iteration
 	Leavers lv;
@@ -225,7 +246,7 @@ void cpic_fft_threads(int64_t mmax, int64_t nymax, int *nt_row, int *nt_col);
 void cpic_fft_blocking(Geo *g, int nt_row, int nt_col);
 void cpic_fft_spread(Geo *g, int P);
 int cpic_fft_blocking_ok(const Geo *g, int nt_row, int nt_col);
-size_t cpic_push_lds(const cpic_dev *d);
+size_t cpic_push_lds(cpic_dev *d);
 int cpic_set_iter(cpic_dev *d, int64_t iter);
 int cpic_solve(cpic_dev *d, int want_energy);
 int cpic_solve_step(cpic_dev *d);

@@ -1,10 +1,11 @@
 // Particle kernels of the gfx950 PIC step.
 //
-// k_push: one workgroup per (tile, species) bucket.  Stages the tile's E
+// k_push: one workgroup per (tile, species) bucket, or several that share one.
+// Stages the tile's E
 // region (tile + 1 cell margin + the CIC +1 node) in LDS -- after a field
 // solve it computes that region from the potential (E = -grad phi,
 // src/field.c:381-406, staged with a one-node halo), so a step never writes
-// or reads a global E array -- streams every particle of the bucket once
+// or reads a global E array -- streams its share of the bucket's particles once
 // (coalesced loads of the state, stored in groups of 64: x[64] y[64] ux[64]
 // uy[64]), and for each particle
 //   gathers E with CIC weights    (interpolate_f2p_E, src/interpolate.c:350-404)
@@ -17,17 +18,18 @@
 //                                  (FP32 push at 2048^2: 5.71 ms per launch with
 //                                  ds_add_f32 on an LDS pointer, 1.80 ms with
 //                                  ds_add_f64)
-//   and writes the tile's stayers to the other particle buffer (the two
-//   buffers swap every step; each wavefront claims its stayers' slots with
-//   one LDS atomic, so no block-wide barrier is needed per chunk) while
+//   and writes it back to its slot, or for large states to the front of the
+//   same bucket in another particle buffer (the two then swap every step; each
+//   wavefront claims its slots with one LDS atomic), while
 //   leavers (particles whose cell moved to another tile: comm_plasma's
-//   collect, src/comm_plasma.c:101-165) wait in an LDS stage and are copied
-//   to a leaver buffer with one global atomic per bucket.
+//   collect, src/comm_plasma.c:101-165) leave a hole, wait in an LDS stage and
+//   are copied to a leaver buffer with one global atomic per workgroup.
 // The LDS rho region is flushed once per workgroup with FP64 global atomics.
-// k_append then places each leaver at the end of its destination bucket
+// k_append then places each leaver in a hole of its destination bucket or
+// behind its last slot
 // (inject_particles, src/comm_plasma.c:358-400) or, when that bucket is full,
-// back into a reserved slot of its source bucket, so no particle is ever lost
-// whatever the capacities; such particles are handled by the slow global
+// in one of the slots that its own bucket's leavers left, so no particle is ever
+// lost whatever the capacities; such particles are handled by the slow global
 // path until the next re-sort.
 //
 // FP64 mode uses the reference's arithmetic bit for bit: positions are
@@ -58,19 +60,21 @@ template <typename T, int U> struct NU { typedef T t __attribute__((ext_vector_t
 struct PushArgs {
 	const Geo *geo;
 	const int *pre_tile;  // [P+1] first global tile of each plasma
-	const int *order;     // [ntiles] tile of each block (cpic_parts_order); k_push:
-	                      // [nb] bucket of each block
+	const int *order;     // [ntiles] tile of each block (cpic_parts_order)
+	const int2 *units;    // k_push: [nunits] (bucket, part | parts << 16) of each block
 	const int *pre_bucket; // [P+1] first global bucket of each plasma
 	int P;
 	int ntiles;           // tiles of the whole batch
 	Buckets bk;
 	Parts p;              // particles read
-	Parts q;              // particles written (the other buffer)
+	Parts q;              // particles written by k_push: p itself or the other buffer
+	int32_t *holes;       // bucket b's ring of holes at its start
 	Leavers lv;
-	int par;              // leaver counter parity
+	int par;              // parity of the step (k_push) or of the last push
 	int first;            // iteration 0: dt' = -dt/2 and no position update
 	const void *E;        // whole batch, plasma p at node0
 	const double *phi;    // potential, whole batch (pushes that compute E)
+	int phi_apart;        // its tile region has LDS of its own
 	double *rho;          // deposit target, whole batch
 	DiagSlot *diag;       // nullable: per-plasma rings of `ring` slots
 	double *dpart;        // with diag: [P][DIAG_SPREAD][DIAG_LINE] accumulators
@@ -135,18 +139,67 @@ static inline int tile_map(int b, int ntiles)
 	return b;
 }
 
-static __device__ __forceinline__ int bucket_n1(const Buckets &bk, int b)
+// A bucket between steps: slots [0, n) but for the gap [gap0, gap1), of which
+// `holes` are empty, listed in the bucket's ring from position head on.  Only
+// buckets in place have holes, only compact ones a gap (in front of particles
+// that came back).
+struct BucketNow { int n, head, holes, gap0, gap1; };
+
+// Position i < 2 cap of a ring of cap entries.
+static __device__ __forceinline__ int ring_at(int i, int cap)
 {
-	int lim = bk.cap[b] - bk.res[b];
-	int n1 = bk.n1[b];
-	return n1 < lim ? n1 : lim;
+	return i >= cap ? i - cap : i;
 }
 
-static __device__ __forceinline__ int64_t bucket_slot(const Buckets &bk, int b,
-		int n1, int j)
+// The state that a step's base and counts come to.  In place, the arrivals took
+// the base's holes first and then slots n, n + 1, ... up to the capacity (those
+// beyond it went back to their sources), and the slots that the step's
+// leavers left are holes.  Compact, they took slots n, n + 1, ... up to the
+// last `out` slots, which those that came back fill from the end.
+static __device__ __forceinline__ BucketNow bucket_after(const BucketBase &v, const BucketCnt &c,
+		int cap, bool compact)
 {
-	int64_t s = bk.start[b];
-	return j < n1 ? s + j : s + (bk.cap[b] - bk.res[b]) + (j - n1);
+	BucketNow r;
+	r.gap0 = r.gap1 = 0;
+	if(compact)
+	{
+		r.head = r.holes = 0;
+		r.n = v.n + min(c.in, cap - c.out - v.n);
+		if(c.back)
+		{
+			r.gap0 = r.n;
+			r.gap1 = cap - c.back;
+			r.n = cap;
+		}
+		return r;
+	}
+	int taken = min(c.in, v.holes);
+	r.n = min(cap, v.n + (c.in - taken));
+	r.head = ring_at(v.head + taken, cap);
+	r.holes = v.holes - taken + c.out - c.back;
+	return r;
+}
+
+// State of bucket b after the last push, whose parity was par.
+static __device__ __forceinline__ BucketNow bucket_now(const Buckets &bk, int par, int b)
+{
+	int64_t i = (int64_t) par * bk.nb + b;
+	return bucket_after(bk.base[i], bk.cnt[i], bk.cap[b], bk.compact);
+}
+
+// Whether slot j < n, with position x, holds a particle.
+template <typename T>
+static __device__ __forceinline__ bool slot_used(const BucketNow &v, int j, T x)
+{
+	return x == x && (j < v.gap0 || j >= v.gap1);
+}
+
+// x of an empty slot.  Particles never hold it: uploads are checked and the
+// push resets a position that is not finite.
+template <typename T>
+static __device__ __forceinline__ T hole_x()
+{
+	return (T) __builtin_nanf("");
 }
 
 // Per-particle state in registers.
@@ -459,16 +512,40 @@ void k_zero(double *__restrict__ p, int64_t n)
 		p[i] = 0.0;
 }
 
+// Position (x, y) of the thread's items in a region of rows of w nodes, taken
+// blockDim.x at a time: one division at the start instead of one per item.
+struct RegionWalk {
+	int w, x, y, sx, sy;
+	__device__ __forceinline__ RegionWalk(int w_) : w(w_)
+	{
+		const int b = (int) blockDim.x;
+		y = (int) threadIdx.x / w;
+		x = (int) threadIdx.x - y * w;
+		sy = b / w;
+		sx = b - sy * w;
+	}
+	__device__ __forceinline__ void next()
+	{
+		x += sx;
+		y += sy;
+		if(x >= w)
+		{
+			x -= w;
+			y++;
+		}
+	}
+};
+
 // Loads the tile's E region into LDS (periodic indexing) and zeroes the
 // LDS rho region.
 template <typename T>
 static __device__ __forceinline__ void tile_setup(const Geo &g, int ox, int oy,
 		const typename V2<T>::t *__restrict__ E, typename V2<T>::t *sE, double *sR)
 {
-	for(int i = threadIdx.x; i < g.W * g.H; i += blockDim.x)
+	RegionWalk r(g.W);
+	for(int i = threadIdx.x; i < g.W * g.H; i += blockDim.x, r.next())
 	{
-		int ly = i / g.W, lx = i - ly * g.W;
-		int gx = wrapi(ox + lx, g.nx), gy = wrapi(oy + ly, g.ny);
+		int gx = wrapi(ox + r.x, g.nx), gy = wrapi(oy + r.y, g.ny);
 		if(sE)
 			sE[i] = E[(int64_t) gy * g.nx + gx];
 		if(sR)
@@ -477,37 +554,51 @@ static __device__ __forceinline__ void tile_setup(const Geo &g, int ox, int oy,
 }
 
 // Computes the tile's E region in LDS from the potential: the region plus a
-// one-node halo of phi is staged in the rho area (row stride W + 2), E
-// follows with the expression of k_efield (src/field.c:381-406), then the rho
-// area is zeroed.
+// one-node halo of phi is staged in sP (row stride W + 2), E
+// follows with the expression of k_efield (src/field.c:381-406), and the rho
+// area is zeroed.  sP is the rho area itself for tiles whose LDS would hold the
+// blocks per CU down; apart from it, the zeroing needs no barrier of its own.
+// In two steps, so that a caller can have other loads in
+// flight meanwhile.
 // The grid sides are powers of two, so "& (n - 1)" wraps any offset.
+static __device__ __forceinline__ void tile_stage_phi(const Geo &g, int ox, int oy,
+		const double *__restrict__ phi, double *sP, double *sR)
+{
+	const int PW = g.W + 2, PH = g.H + 2;
+	RegionWalk r(PW);
+	for(int i = threadIdx.x; i < PW * PH; i += blockDim.x, r.next())
+	{
+		int gx = (ox - 1 + r.x) & (g.nx - 1), gy = (oy - 1 + r.y) & (g.ny - 1);
+		sP[i] = phi[(int64_t) gy * g.nx + gx];
+		if(sP != sR && i < g.W * g.H)
+			sR[i] = 0.0;
+	}
+}
+
 template <typename T>
-static __device__ __forceinline__ void tile_setup_phi(const Geo &g, int ox, int oy,
-		const double *__restrict__ phi, typename V2<T>::t *sE, double *sR)
+static __device__ __forceinline__ void tile_E_of_phi(const Geo &g, typename V2<T>::t *sE,
+		const double *sP, double *sR)
 {
 	typedef typename V2<T>::t T2;
-	const int PW = g.W + 2, PH = g.H + 2;
-	for(int i = threadIdx.x; i < PW * PH; i += blockDim.x)
-	{
-		int ly = i / PW, lx = i - ly * PW;
-		int gx = (ox - 1 + lx) & (g.nx - 1), gy = (oy - 1 + ly) & (g.ny - 1);
-		sR[i] = phi[(int64_t) gy * g.nx + gx];
-	}
+	const int PW = g.W + 2;
+	RegionWalk r(g.W);
 	__syncthreads();
-	for(int i = threadIdx.x; i < g.W * g.H; i += blockDim.x)
+	for(int i = threadIdx.x; i < g.W * g.H; i += blockDim.x, r.next())
 	{
-		int ly = i / g.W, lx = i - ly * g.W;
-		int c = (ly + 1) * PW + lx + 1;
-		double ey = (sR[c - PW] - sR[c + PW]) / (2 * g.dy);
-		double ex = (sR[c - 1] - sR[c + 1]) / (2 * g.dx);
+		int c = (r.y + 1) * PW + r.x + 1;
+		double ey = (sP[c - PW] - sP[c + PW]) / (2 * g.dy);
+		double ex = (sP[c - 1] - sP[c + 1]) / (2 * g.dx);
 		T2 v;
 		v.x = ex;
 		v.y = ey;
 		sE[i] = v;
 	}
-	__syncthreads();
-	for(int i = threadIdx.x; i < g.W * g.H; i += blockDim.x)
-		sR[i] = 0.0;
+	if(sP == sR)
+	{
+		__syncthreads();
+		for(int i = threadIdx.x; i < g.W * g.H; i += blockDim.x)
+			sR[i] = 0.0;
+	}
 }
 
 // Adds the LDS rho region into the global rho with FP64 atomics.
@@ -515,13 +606,13 @@ template <typename T>
 static __device__ __forceinline__ void tile_flush(const Geo &g, int ox, int oy, const double *sR,
 		double *__restrict__ rho)
 {
-	for(int i = threadIdx.x; i < g.W * g.H; i += blockDim.x)
+	RegionWalk r(g.W);
+	for(int i = threadIdx.x; i < g.W * g.H; i += blockDim.x, r.next())
 	{
 		double v = sR[i];
 		if(v != 0.0)
 		{
-			int ly = i / g.W, lx = i - ly * g.W;
-			int gx = wrapi(ox + lx, g.nx), gy = wrapi(oy + ly, g.ny);
+			int gx = wrapi(ox + r.x, g.nx), gy = wrapi(oy + r.y, g.ny);
 			unsafeAtomicAdd(&rho[(int64_t) gy * g.nx + gx], (double) v);
 		}
 	}
@@ -595,100 +686,77 @@ static __device__ __forceinline__ bool push_one(const Geo &g, const typename V2<
 	return true;
 }
 
-// Loads the chunk of U*NT particles starting at bucket index base (NT
-// threads): thread tid takes base + U*tid + u with vector loads when U = 4
-// and the chunk lies in the bucket's first segment, else base + u*NT + tid
-// (coalesced loads either way; every slot of the chunk exactly once).
-template <typename T, bool IDS, int U, int NT>
-static __device__ __forceinline__ void load_chunk(const Parts &p, int64_t bstart, int n1,
-		int seg2, int ntot, int base, int tid, PState<T> *q, bool *act)
-{
-	const GLB_AS T *pb = bucket_base<T>(p, bstart);
-	if(U == 4 && base + U * NT <= n1)
+// Slots of a thread's U particles in a chunk of U*nt slots.  In a full chunk:
+// NV vectors of V slots, vector v at base + v*V*nt + V*tid, V slots filling 16
+// bytes, or single slots where a thread's particles fill less (8-byte vectors
+// of FP32 pairs were 4 % slower than single slots).  In a bucket's last, partly
+// filled chunk single slots, nt apart, so that its particles spread over the
+// wavefronts instead of U to a thread.
+template <typename T, int U> struct ChunkMap {
+	static constexpr int V = U * sizeof(T) < 16 ? 1 : 16 / (int) sizeof(T);
+	static constexpr int NV = U / V;
+	typedef typename NU<T, V>::t vec;
+	// bucket slot of the thread's u-th particle in the chunk at base
+	static __device__ __forceinline__ int slot(int base, int tid, int u, int nt, bool full)
 	{
-		// the whole chunk lies in the first segment (the usual case): thread
-		// tid takes the U consecutive slots base + U*tid ... (U divides the
-		// group of 64, so they are contiguous), one vector load per component.
-		// Measured with U = 4 only: with U = 2 (two-element vectors) the push
-		// was 4 % slower than with the per-slot loads below.
-		typedef typename NU<T, U>::t VU;
-		const int j0 = base + U * tid;
-		const GLB_AS VU *r = (const GLB_AS VU *) at_byte(pb, pslot_byte<T>(j0));
-		VU vx = r[0], vy = r[PGROUP / U], vux = r[2 * PGROUP / U], vuy = r[3 * PGROUP / U];
-#pragma unroll
-		for(int u = 0; u < U; u++)
-		{
-			act[u] = true;
-			q[u].x = vx[u];
-			q[u].y = vy[u];
-			q[u].ux = vux[u];
-			q[u].uy = vuy[u];
-			if(IDS)
-				q[u].id = gptr<int64_t>(p.id)[bstart + j0 + u];
-		}
-		return;
+		return full ? base + (u / V) * (V * nt) + V * tid + u % V : base + u * nt + tid;
 	}
-#pragma unroll
-	for(int u = 0; u < U; u++)
-	{
-		int j = base + u * NT + tid;
-		act[u] = j < ntot;
-		int jj = j + (j >= n1 ? seg2 : 0);
-		if(act[u])
-		{
-			// global-address-space loads (see load_p)
-			const GLB_AS T *r = at_byte(pb, pslot_byte<T>(jj));
-			q[u].x = r[0];
-			q[u].y = r[PGROUP];
-			q[u].ux = r[2 * PGROUP];
-			q[u].uy = r[3 * PGROUP];
-			if(IDS)
-				q[u].id = gptr<int64_t>(p.id)[bstart + jj];
-		}
-	}
-}
+};
 
-// Fused gather + push + wrap + deposit + tile compaction.  Each thread
-// handles U particles per chunk (particle base + u*256 + tid), all loads of
-// a chunk issued before any of them is used, so a workgroup keeps U*256
-// particles of HBM reads in flight.  Stayers go to the front of the same
-// bucket in the other buffer (a.q), each wavefront claiming its slots with
-// one LDS atomic (their order within the bucket is not kept); leavers go
-// to the leaver buffer with one atomic per wavefront.
+// Fused gather + push + wrap + deposit.  A workgroup takes a range
+// of whole chunks (part of parts) of one bucket; each thread handles U
+// particles per chunk, all loads of a chunk issued before any of them is
+// used.  In place, it writes them back to the same slots with whole vector
+// stores, so
+// nothing is claimed, compacted or moved for the particles that stay, and
+// workgroups that share a bucket need no agreement on its slots; a
+// particle that left the tile leaves a hole (x = NaN) whose slot goes to the
+// bucket's ring.  COMPACT, the stayers go to the front of the same bucket in the
+// other buffer (their order is not kept) and one workgroup takes a whole bucket.
+// Leavers go to the leaver buffer.
+//
+// Bound by HBM, for small states by the memory-side cache (256 MB) and, with
+// few particles per bucket, by each workgroup's set-up and flush.  In place
+// (a.q = a.p) the state's footprint is halved, and the units run in opposite
+// directions in consecutive steps, so that a step meets the last-touched state
+// first: a stream of this pattern moved 268 MB of state in 76 us in place and
+// 107 us from buffer to buffer, and 537 MB in 165 us in place with the
+// reversal, 208 us without it and 205 us between buffers.  push_in_place()
+// says up to which size.  Push per launch, compact with one workgroup per
+// bucket -> in place: FP32 256^2, 4.2 M particles 60.5 -> 35.4 us; FP64 512^2 with
+// Bz, 16.8 M 242 -> 195 us; FP64 33.6 M 481 -> 423 us; FP32 512^2, 16.8 M 144 ->
+// 112 us (U = 2), 130 -> 108 us (U = 4); FP32 ensemble of 24 plasmas, 46 M 321 ->
+// 302 us.
 //
 // Waves per SIMD the register allocation of k_push must allow.  Measured at
-// 2048^2, 64 ppc: the FP32 kernel gains ~3 % from 6 waves (U = 2, now 73
-// VGPRs; 7 waves gain nothing), the FP64 kernel loses from any bound (its
-// state is twice the size); bounding the FP32 U = 4 kernel (then 95 VGPRs,
-// now 93) to 6 waves spilled and lost 12 %.
+// 2048^2, 64 ppc: the FP32 kernel gains ~3 % from 6 waves (U = 2), the FP64
+// kernel loses from any bound (its state is twice the size); bounding the
+// FP32 U = 4 kernel to 6 waves spilled and lost 12 %.
 #ifndef PUSH_MIN_WAVES_F32
 #define PUSH_MIN_WAVES_F32 6
 #endif
-// Threads per k_push workgroup.  512 (half the chunks per bucket; the
-// compiler then holds the FP32 kernel to 81 VGPRs) measured slower at
-// 2048^2: FP32 push 1.89 vs 1.74 ms, FP64 3.78 vs 3.29 ms.
+// Threads per k_push workgroup.
 #ifndef PUSH_BLOCK
 #define PUSH_BLOCK CPIC_BLOCK
 #endif
 
-
-
-// Leavers of one bucket wait in LDS and are placed in the leaver buffer with
-// one global atomic per bucket: a counter shared by every workgroup, hit once
+// Leavers of one workgroup wait in LDS and are placed in the leaver buffer with
+// one global atomic per workgroup: a counter shared by every workgroup, hit once
 // per wavefront with a leaver, serialises in one L2 channel and stalls the
 // wavefront until it returns.  A wavefront whose leavers no longer fit in the
-// stage claims its slots with its own global atomic.
+// stage claims its slots with its own global atomics.
 #ifndef LV_STAGE
 #define LV_STAGE 256
 #endif
 template <typename T, bool IDS, bool PE> struct LvStage {
 	T x[LV_STAGE], y[LV_STAGE], ux[LV_STAGE], uy[LV_STAGE];
-	int dst[LV_STAGE];
+	int dst[LV_STAGE], slot[LV_STAGE];
 	int64_t id[IDS ? LV_STAGE : 1];
 	double Ex[PE ? LV_STAGE : 1], Ey[PE ? LV_STAGE : 1];
 	int n;        // records claimed (may pass LV_STAGE)
 	int cut;      // first record of the wavefront that did not fit
 	int base;     // first leaver-buffer slot of the staged records
+	int hole;     // their first position among the step's new holes
 };
 
 // An FP32 leaver (coordinates relative to destination bucket ndst) put back
@@ -710,23 +778,31 @@ static __device__ __forceinline__ void back_to_tile(const Geo &g, int ndst, int 
 	q.y = (T) ((float) q.y + (float) dty);
 }
 
+// Unit of block b of n: the other way round every other step in place (see
+// above), the XCD of a block (b mod 8) kept.
+static __device__ __forceinline__ int unit_of_block(int b, int n, int par)
+{
+	if(!par)
+		return b;
+	return (n & 7) == 0 ? (n - 8 - (b & ~7)) + (b & 7) : n - 1 - b;
+}
+
 // EPHI: the tile's E comes from the potential (the E array is stale).
-template <typename T, bool IDS, bool PE, int U, bool EPHI>
+// COMPACT: the buckets are kept compact (one workgroup per bucket).
+template <typename T, bool IDS, bool PE, int U, bool EPHI, bool COMPACT>
 __global__ __launch_bounds__(PUSH_BLOCK, sizeof(T) == 4 && U == 2 && !IDS && !PE ? PUSH_MIN_WAVES_F32 : 1)
 void k_push(PushArgs a)
 {
 	typedef typename V2<T>::t T2;
+	typedef ChunkMap<T, U> Map;
+	constexpr int V = Map::V, NV = Map::NV, CHUNK = U * PUSH_BLOCK;
 	extern __shared__ unsigned char smem[];
-	__shared__ int s_kcount;
-	__shared__ int s_w;
 	__shared__ LvStage<T, IDS, PE> s_lv;
+	__shared__ int s_w;        // COMPACT: slots taken in the other buffer
 
-	// one (tile, species) bucket per block: the tile's species run as
-	// separate blocks (fewer chunks per block than one block per tile: a
-	// stream of this access pattern measured 1.60 ms at 8 chunks per block
-	// and 1.55 ms at 4; the push 2.4 % faster in FP32, 3.4 % in FP64)
-	const int unit = a.order[blockIdx.x];
-	const int pl = find_plasma(a.pre_bucket, a.P, unit);
+	const int2 unit = a.units[unit_of_block(blockIdx.x, gridDim.x, COMPACT ? 0 : a.par)];
+	const int b = unit.x, part = unit.y & 0xffff, parts = unit.y >> 16;
+	const int pl = find_plasma(a.pre_bucket, a.P, b);
 	// the plasma's table entry, read once into registers (a reference into
 	// global memory would be re-read after every particle store); the
 	// per-species arrays are read through gp
@@ -734,8 +810,8 @@ void k_push(PushArgs a)
 	const Geo g = *gp;
 	T2 *sE = (T2 *) smem;
 	double *sR = (double *) (smem + sizeof(T2) * g.W * g.H);
+	double *sP = a.phi_apart ? sR + g.W * g.H : sR;
 
-	const int b = unit;
 	const int tile = (b - g.bucket0) / g.ns;
 	const int s = b - g.bucket0 - tile * g.ns;
 	int tix = tile & (g.ntx - 1), tiy = tile >> g.lgntx;
@@ -749,55 +825,138 @@ void k_push(PushArgs a)
 	const float dtdx = (float) (dtp / g.dx), dtdy = (float) (dtp / g.dy);
 	// read here, used at the end: its load latency then overlaps the work
 	const long long iter = a.diag ? a.st->iter : -1;
+	if(a.diag && blockIdx.x == 0 && tid == 0)
+		*a.diag_iter = iter;
+
+	// the bucket's state after the last step (loaded here, waited for after
+	// the potential's loads are out)
+	const int64_t last = (int64_t) (1 - a.par) * a.bk.nb + b;
+	const BucketBase lbase = a.bk.base[last];
+	const BucketCnt lcnt = a.bk.cnt[last];
+	const int64_t lstart = a.bk.start[b];
+	const int lcap = a.bk.cap[b];
 
 	if(EPHI)
-		tile_setup_phi<T>(g, ox, oy, phi, sE, sR);
+		tile_stage_phi(g, ox, oy, phi, sP, sR);
 	else
 		tile_setup<T>(g, ox, oy, E, sE, sR);
 	if(tid == 0)
 	{
-		s_kcount = 0;
-		s_w = 0;
 		s_lv.n = 0;
 		s_lv.cut = LV_STAGE;
+		s_w = 0;
 	}
-	__syncthreads();
+
+	const int64_t bstart = uniform(lstart);
+	const int cap = uniform(lcap);
+	BucketNow bn = bucket_after(lbase, lcnt, lcap, COMPACT);
+	bn.n = uniform(bn.n);
+	bn.head = uniform(bn.head);
+	bn.holes = uniform(bn.holes);
+	bn.gap0 = uniform(bn.gap0);
+	bn.gap1 = uniform(bn.gap1);
+	BucketCnt *cnt = &a.bk.cnt[(int64_t) a.par * a.bk.nb + b];
+	// part 0 records it as this step's base (compact buckets get theirs at
+	// the end)
+	if(part == 0 && tid == 0)
+	{
+		BucketBase v = {COMPACT ? 0 : bn.n, bn.head, bn.holes, 0};
+		a.bk.base[(int64_t) a.par * a.bk.nb + b] = v;
+	}
+	int32_t *ring = a.holes + bstart;
+	const int ring0 = ring_at(bn.head + bn.holes, cap);   // first new hole
+	// this part's chunks
+	const int nchunks = (bn.n + CHUNK - 1) / CHUNK;
+	const int end = (int) ((int64_t) nchunks * (part + 1) / parts) * CHUNK;
+	int base = (int) ((int64_t) nchunks * part / parts) * CHUNK;
+	if(base >= end)
+		return;
 
 	double ke = 0.0, mpx = 0.0, mpy = 0.0;
 	bool bad = false, nan_ = false;
-
-	const int64_t bstart = uniform(a.bk.start[b]);
-	const int cap = uniform(a.bk.cap[b]), res = uniform(a.bk.res[b]);
-	const int n1 = min(uniform(a.bk.n1[b]), cap - res);
-	const int ntot = n1 + uniform(a.bk.n2[b]);
-	const int seg2 = cap - res - n1;      // slot = j + seg2 for j >= n1
 	const SpeciesK<T> sk = species_k<T>(*gp, s, dtp);
+	const GLB_AS T *pb = bucket_base<T>(a.p, bstart);
+	GLB_AS T *qb = (GLB_AS T *) bucket_base<T>(a.q, bstart);
+	if(EPHI)
+		tile_E_of_phi<T>(g, sE, sP, sR);
+	__syncthreads();
 
-	for(int base = 0; base < ntot; base += U * PUSH_BLOCK)
+	for(; base < end; base += CHUNK)
 	{
 		PState<T> q[U];
-		bool act[U], leave[U];
-		int ndst[U];
-		load_chunk<T, IDS, U, PUSH_BLOCK>(a.p, bstart, n1, seg2, ntot, base, tid, q, act);
+		bool act[U];
+		const bool full = base + CHUNK <= bn.n && (!COMPACT || bn.gap1 == 0);
+		auto load_chunk = [&]() {
+			if(full)
+			{
 #pragma unroll
-		for(int u = 0; u < U; u++)
-		{
+				for(int v = 0; v < NV; v++)
+				{
+					const int j = Map::slot(base, tid, v * V, PUSH_BLOCK, true);
+					const GLB_AS typename Map::vec *r =
+						(const GLB_AS typename Map::vec *) at_byte(pb, pslot_byte<T>(j));
+					typename Map::vec vx = r[0], vy = r[PGROUP / V];
+					typename Map::vec vux = r[2 * PGROUP / V], vuy = r[3 * PGROUP / V];
+#pragma unroll
+					for(int i = 0; i < V; i++)
+					{
+						const int u = v * V + i;
+						q[u].x = vx[i];
+						q[u].y = vy[i];
+						q[u].ux = vux[i];
+						q[u].uy = vuy[i];
+						act[u] = COMPACT || vx[i] == vx[i];   // not a hole
+					}
+				}
+				return;
+			}
+#pragma unroll
+			for(int u = 0; u < U; u++)
+			{
+				const int j = Map::slot(base, tid, u, PUSH_BLOCK, false);
+				act[u] = j < bn.n && (!COMPACT || j < bn.gap0 || j >= bn.gap1);
+				if(act[u])
+				{
+					const GLB_AS T *r = at_byte(pb, pslot_byte<T>(j));
+					q[u].x = r[0];
+					q[u].y = r[PGROUP];
+					q[u].ux = r[2 * PGROUP];
+					q[u].uy = r[3 * PGROUP];
+				}
+			}
+			if(!COMPACT)
+			{
+#pragma unroll
+				for(int u = 0; u < U; u++)
+					act[u] = act[u] && q[u].x == q[u].x;          // not a hole
+			}
+		};
+		load_chunk();
+		// wait for all of the chunk's loads (vmcnt 0) before its first particle:
+		// one burst per chunk rather than loads that trail into the arithmetic.
+		// Compact FP32 push of 134 M particles, U = 4: 921 -> 888 us, U = 2: 897 ->
+		// 886; FP32 in place at 512^2 (16.8 M), U = 2: 118 -> 112; others unchanged
+		__builtin_amdgcn_s_waitcnt(0x0f70);
+		bool leave[U];
+		int ndst[U];
+		auto push_u = [&](int u) {
 			leave[u] = false;
 			ndst[u] = 0;
 			if(act[u])
 				leave[u] = push_one<T, EPHI>(g, sE, E, phi, sR, rho, tile, ox, oy, s, sk, set_r,
 						dtp, dtdx, dtdy, q[u], ndst[u], ke, mpx, mpy, bad, nan_);
-		}
-		// leavers: staged in LDS (one LDS atomic per wavefront); once
-		// the stage is full, placed directly (one global atomic each)
-#pragma unroll
-		for(int u = 0; u < U; u++)
-		{
+		};
+		// leavers are staged in LDS (one LDS atomic per wavefront) or, once the
+		// stage is full, placed directly (global atomics each)
+		auto stage_u = [&](int u) {
 			unsigned long long lm = __ballot(leave[u]);
 			if(lm)
 			{
+				const int slot = Map::slot(base, tid, u, PUSH_BLOCK, full);
 				int lcnt = __popcll(lm);
 				int sb = 0;
+				if(IDS && leave[u])
+					q[u].id = gptr<int64_t>(a.p.id)[bstart + slot];
 				if(lane == 0)
 					sb = atomicAdd(&s_lv.n, lcnt);
 				sb = __builtin_amdgcn_readfirstlane(sb);
@@ -811,6 +970,7 @@ void k_push(PushArgs a)
 						s_lv.ux[k] = q[u].ux;
 						s_lv.uy[k] = q[u].uy;
 						s_lv.dst[k] = ndst[u];
+						s_lv.slot[k] = slot;
 						if(IDS)
 							s_lv.id[k] = q[u].id;
 						if(PE)
@@ -844,74 +1004,138 @@ void k_push(PushArgs a)
 						}
 					}
 					unsigned long long placed = __ballot(leave[u]);
-					if(lane == 0 && placed)
-						atomicAdd(&s_kcount, __popcll(placed));
+					if(placed)
+					{
+						int hb = 0;
+						if(lane == 0)
+							hb = atomicAdd(&cnt->out, __popcll(placed));
+						hb = __builtin_amdgcn_readfirstlane(hb);
+						if(leave[u] && !COMPACT)
+							ring[ring_at(ring0 + hb + lanes_below(placed), cap)] = slot;
+					}
 				}
 			}
-		}
-		// stayers: one LDS atomic per wavefront and chunk claims their
-		// slots in the other buffer for all U rounds (order within the
-		// bucket is not kept)
-		unsigned long long smks[U];
-		int wbase = 0, wtot = 0;
+			if(PE && act[u] && !leave[u])
+			{
+				const int j = Map::slot(base, tid, u, PUSH_BLOCK, full);
+				a.p.Ex[bstart + j] = q[u].Ex;
+				a.p.Ey[bstart + j] = q[u].Ey;
+			}
+			if(!COMPACT && leave[u])
+				q[u].x = hole_x<T>();
+		};
+
+		// in place, a leaver is staged right after its push (fewer registers
+		// live: 91 instead of 101 for FP32, U = 4, before the loads moved into
+		// the loop); compacting needs all U flags anyway
+		if(COMPACT)
+		{
 #pragma unroll
-		for(int u = 0; u < U; u++)
-		{
-			smks[u] = __ballot(act[u] && !leave[u]);
-			wtot += __popcll(smks[u]);
-		}
-		if(wtot)
-		{
-			if(lane == 0)
-				wbase = atomicAdd(&s_w, wtot);
-			wbase = __builtin_amdgcn_readfirstlane(wbase);
-		}
+			for(int u = 0; u < U; u++)
+				push_u(u);
 #pragma unroll
-		for(int u = 0; u < U; u++)
+			for(int u = 0; u < U; u++)
+				stage_u(u);
+		}
+		else
 		{
-			unsigned long long smk = smks[u];
-			int wb = wbase;
-			wbase += __popcll(smk);
-			if(smk)
+#pragma unroll
+			for(int u = 0; u < U; u++)
+			{
+				push_u(u);
+				stage_u(u);
+			}
+		}
+		if(COMPACT)
+		{
+			// one LDS atomic per wavefront and chunk claims slots in the
+			// other buffer for all U rounds
+			unsigned long long smk[U];
+			int wb = 0, wtot = 0;
+#pragma unroll
+			for(int u = 0; u < U; u++)
+			{
+				smk[u] = __ballot(act[u] && !leave[u]);
+				wtot += __popcll(smk[u]);
+			}
+			if(wtot)
+			{
+				if(lane == 0)
+					wb = atomicAdd(&s_w, wtot);
+				wb = __builtin_amdgcn_readfirstlane(wb);
+			}
+#pragma unroll
+			for(int u = 0; u < U; u++)
 			{
 				if(act[u] && !leave[u])
 				{
-					int jj = wb + lanes_below(smk);
-					GLB_AS T *r = at_byte(bucket_base<T>(a.q, bstart), pslot_byte<T>(jj));
+					GLB_AS T *r = at_byte(qb, pslot_byte<T>(wb + lanes_below(smk[u])));
 					r[0] = q[u].x;
 					r[PGROUP] = q[u].y;
 					r[2 * PGROUP] = q[u].ux;
 					r[3 * PGROUP] = q[u].uy;
-					if(IDS)
-						a.q.id[bstart + jj] = q[u].id;
-					if(PE)
-					{
-						a.q.Ex[bstart + jj] = q[u].Ex;
-						a.q.Ey[bstart + jj] = q[u].Ey;
-					}
 				}
+				wb += __popcll(smk[u]);
 			}
+		}
+		// every slot back where it was; a leaver's becomes a hole
+		else if(full)
+		{
+#pragma unroll
+			for(int v = 0; v < NV; v++)
+			{
+				const int j = Map::slot(base, tid, v * V, PUSH_BLOCK, true);
+				typename Map::vec vx, vy, vux, vuy;
+#pragma unroll
+				for(int i = 0; i < V; i++)
+				{
+					const int u = v * V + i;
+					vx[i] = q[u].x;
+					vy[i] = q[u].y;
+					vux[i] = q[u].ux;
+					vuy[i] = q[u].uy;
+				}
+				GLB_AS typename Map::vec *r =
+					(GLB_AS typename Map::vec *) at_byte(qb, pslot_byte<T>(j));
+				r[0] = vx;
+				r[PGROUP / V] = vy;
+				r[2 * PGROUP / V] = vux;
+				r[3 * PGROUP / V] = vuy;
+			}
+		}
+		else
+		{
+#pragma unroll
+			for(int u = 0; u < U; u++)
+				if(act[u])
+				{
+					GLB_AS T *r = at_byte(qb,
+							pslot_byte<T>(Map::slot(base, tid, u, PUSH_BLOCK, false)));
+					r[0] = q[u].x;
+					r[PGROUP] = q[u].y;
+					r[2 * PGROUP] = q[u].ux;
+					r[3 * PGROUP] = q[u].uy;
+				}
 		}
 	}
 
-	// the bucket's staged leavers: one global atomic claims their slots
+	// the staged leavers: one global atomic claims their slots, one their
+	// holes' places in the ring; the flush runs meanwhile
 	__syncthreads();
-	if(tid == 0)
+	const int staged = min(s_lv.n, s_lv.cut);
+	if(tid == 0 && staged > 0)
 	{
-		int nst = min(s_lv.n, s_lv.cut);
-		s_lv.n = nst;
-		s_lv.base = nst > 0 ? atomicAdd(&a.lv.count[a.par], nst) : 0;
-		if(nst > 0)
-		{
-			int64_t room = a.lv.cap - (int64_t) s_lv.base;
-			s_kcount += (int) (room <= 0 ? 0 : room < nst ? room : nst);
-		}
+		s_lv.base = atomicAdd(&a.lv.count[a.par], staged);
+		int64_t room = a.lv.cap - (int64_t) s_lv.base;
+		int placed = (int) (room <= 0 ? 0 : room < staged ? room : staged);
+		s_lv.hole = placed > 0 ? atomicAdd(&cnt->out, placed) : 0;
 	}
-	__syncthreads();
+	tile_flush<T>(g, ox, oy, sR, rho);
+	if(staged > 0)
 	{
-		const int nst = s_lv.n;
+		__syncthreads();
 		const int64_t lb0 = s_lv.base;
-		for(int k = tid; k < nst; k += PUSH_BLOCK)
+		for(int k = tid; k < staged; k += PUSH_BLOCK)
 		{
 			PState<T> lq;
 			lq.x = s_lv.x[k];
@@ -921,25 +1145,30 @@ void k_push(PushArgs a)
 			lq.id = IDS ? s_lv.id[k] : 0;
 			lq.Ex = PE ? s_lv.Ex[k] : 0.0;
 			lq.Ey = PE ? s_lv.Ey[k] : 0.0;
-			int nd = s_lv.dst[k];
+			int nd = s_lv.dst[k], slot = s_lv.slot[k];
 			if(lb0 + k < a.lv.cap)
+			{
 				store_l<T>(a.lv, lb0 + k, lq, IDS, PE, nd, b);
+				if(!COMPACT)
+					ring[ring_at(ring0 + s_lv.hole + k, cap)] = slot;
+			}
 			else
 			{
 				// no room: stays in this bucket (misplaced)
 				back_to_tile<T>(g, nd, ox, oy, lq);
-				int w = atomicAdd(&s_w, 1);
-				store_p<T>(a.q, bstart + w, lq, IDS, PE);
+				if(COMPACT)
+					slot = atomicAdd(&s_w, 1);
+				store_p<T>(a.q, bstart + slot, lq, IDS, PE);
 				atomicAdd(&a.ctr->misplaced, 1ull);
 			}
 		}
 	}
-	__syncthreads();
-	if(tid == 0)
+
+	if(COMPACT)
 	{
-		a.bk.n1[b] = s_w;
-		a.bk.res[b] = s_kcount;
-		a.bk.n2[b] = 0;
+		__syncthreads();
+		if(tid == 0)
+			a.bk.base[(int64_t) a.par * a.bk.nb + b].n = s_w;
 	}
 
 	if(bad)
@@ -947,10 +1176,6 @@ void k_push(PushArgs a)
 	if(nan_)
 		atomicOr(a.derr, CPIC_DERR_NAN);
 
-	tile_flush<T>(g, ox, oy, sR, rho);
-
-	if(a.diag && blockIdx.x == 0 && tid == 0)
-		*a.diag_iter = iter;
 	if(iter >= 0)
 	{
 		// wavefront sums, then one of the plasma's DIAG_SPREAD accumulators
@@ -1012,14 +1237,16 @@ void k_deposit(PushArgs a)
 	for(int s = 0; s < g.ns; s++)
 	{
 		int b = g.bucket0 + tile * g.ns + s;
-		int n1 = bucket_n1(a.bk, b), ntot = n1 + a.bk.n2[b];
+		const BucketNow v = bucket_now(a.bk, a.par, b);
 		T vq = (T) (-gp->q[s] / g.e0);
-		for(int j = threadIdx.x; j < ntot; j += CPIC_BLOCK)
+		for(int j = threadIdx.x; j < v.n; j += CPIC_BLOCK)
 		{
-			int64_t slot = bucket_slot(a.bk, b, n1, j);
+			int64_t slot = a.bk.start[b] + j;
 			CellPos c;
-			T rx, ry;
-			locate(g, ox, oy, p_x<T>(a.p, slot), p_y<T>(a.p, slot), c, rx, ry);
+			T rx, ry, x = p_x<T>(a.p, slot);
+			if(!slot_used(v, j, x))
+				continue;
+			locate(g, ox, oy, x, p_y<T>(a.p, slot), c, rx, ry);
 			deposit<T>(g, sR, rho, c, rx, ry, vq);
 		}
 	}
@@ -1046,13 +1273,15 @@ void k_gather(PushArgs a)
 	for(int s = 0; s < g.ns; s++)
 	{
 		int b = g.bucket0 + tile * g.ns + s;
-		int n1 = bucket_n1(a.bk, b), ntot = n1 + a.bk.n2[b];
-		for(int j = threadIdx.x; j < ntot; j += CPIC_BLOCK)
+		const BucketNow v = bucket_now(a.bk, a.par, b);
+		for(int j = threadIdx.x; j < v.n; j += CPIC_BLOCK)
 		{
-			int64_t slot = bucket_slot(a.bk, b, n1, j);
+			int64_t slot = a.bk.start[b] + j;
 			CellPos c;
-			T rx, ry, ex, ey;
-			locate(g, ox, oy, p_x<T>(a.p, slot), p_y<T>(a.p, slot), c, rx, ry);
+			T rx, ry, ex, ey, x = p_x<T>(a.p, slot);
+			if(!slot_used(v, j, x))
+				continue;
+			locate(g, ox, oy, x, p_y<T>(a.p, slot), c, rx, ry);
 			gather<T, false>(g, sE, E, (const double *) NULL, c, rx, ry, ex, ey);
 			a.p.Ex[slot] = (double) ex;
 			a.p.Ey[slot] = (double) ey;
@@ -1064,16 +1293,18 @@ void k_gather(PushArgs a)
 // within 1-2 % at 2048^2; 2 leaves room for the FP32 occupancy bound above),
 // 4 on request (cpic_dev_desc_t.ppt, chosen by the autotuner)
 
-// Places leavers in their destination bucket, or back in the reserved
-// slots of their source bucket when the destination is full.  The last
-// kernel of a step: it also advances the device step counter, and with diag
+// Places leavers in their destination bucket (in its holes, then behind its
+// slots), or back in a slot that their source bucket's leavers left when the
+// destination is full.  The last
+// kernel of a step: it also advances the device step counter, clears the
+// next step's bucket counts, and with diag
 // adds the push's kinetic and momentum accumulators into each plasma's
 // diagnostic slot (of the iteration the push recorded, so not racing the
 // counter's advance).
 template <typename T, bool IDS, bool PE>
 __global__ __launch_bounds__(CPIC_BLOCK)
 void k_append(const Geo *__restrict__ geo, const int *__restrict__ pre_bucket, int P,
-		Buckets bk, Parts p, Leavers lv, int par, Counters *ctr, StepState *st,
+		Buckets bk, Parts p, const int32_t *__restrict__ holes, Leavers lv, int par, Counters *ctr, StepState *st,
 		double *__restrict__ dpart, const long long *__restrict__ diag_iter,
 		DiagSlot *__restrict__ diag, int ring)
 {
@@ -1092,6 +1323,12 @@ void k_append(const Geo *__restrict__ geo, const int *__restrict__ pre_bucket, i
 		lv.count[1 - par] = 0;
 		st->iter += 1;
 	}
+	for(int64_t i = blockIdx.x * (int64_t) blockDim.x + threadIdx.x; i < bk.nb;
+			i += (int64_t) gridDim.x * blockDim.x)
+	{
+		const BucketCnt z = {0, 0, 0, 0};
+		bk.cnt[(int64_t) (1 - par) * bk.nb + i] = z;
+	}
 	for(int64_t i = blockIdx.x * (int64_t) blockDim.x + threadIdx.x; i < n;
 			i += (int64_t) gridDim.x * blockDim.x)
 	{
@@ -1108,14 +1345,37 @@ void k_append(const Geo *__restrict__ geo, const int *__restrict__ pre_bucket, i
 			q.Ex = lv.Ex[i];
 			q.Ey = lv.Ey[i];
 		}
-		int slot = atomicAdd(&bk.n1[d], 1);
+		const int64_t o = (int64_t) par * bk.nb;
+		const BucketBase v = bk.base[o + d];
+		const int cap = bk.cap[d];
+		int k = atomicAdd(&bk.cnt[o + d].in, 1);
 		int64_t at;
-		if(slot < bk.cap[d] - bk.res[d])
-			at = bk.start[d] + slot;
+		bool back = false;      // destination full
+		if(bk.compact)
+		{
+			back = v.n + k >= cap - bk.cnt[o + d].out;
+			at = bk.start[d] + v.n + k;
+			if(back)
+				at = bk.start[s] + bk.cap[s] - 1 - atomicAdd(&bk.cnt[o + s].back, 1);
+		}
+		else if(k < v.holes)
+			at = bk.start[d] + holes[bk.start[d] + ring_at(v.head + k, cap)];
 		else
 		{
-			int s2 = atomicAdd(&bk.n2[s], 1);
-			at = bk.start[s] + (bk.cap[s] - bk.res[s]) + s2;
+			back = v.n + (k - v.holes) >= cap;
+			at = bk.start[d] + v.n + (k - v.holes);
+			if(back)
+			{
+				// the last of the holes that the source's leavers made
+				const BucketBase vs = bk.base[o + s];
+				const int caps = bk.cap[s];
+				int r = atomicAdd(&bk.cnt[o + s].back, 1);
+				int h = ring_at(vs.head + vs.holes, caps) + bk.cnt[o + s].out - 1 - r;
+				at = bk.start[s] + holes[bk.start[s] + ring_at(h, caps)];
+			}
+		}
+		if(back)
+		{
 			if(sizeof(T) == 4)
 			{
 				const Geo &g = geo[find_plasma(pre_bucket, P, d)];
@@ -1161,7 +1421,7 @@ static __device__ __forceinline__ int find_seg(const int64_t *__restrict__ segpr
 template <typename T>
 __global__ __launch_bounds__(CPIC_BLOCK)
 void k_hist_layout(const Geo *__restrict__ geo, const int *__restrict__ pre_bucket, int P,
-		Buckets bk, Parts p, const int *__restrict__ skip, int *__restrict__ cnt)
+		Buckets bk, int par, Parts p, const int *__restrict__ skip, int *__restrict__ cnt)
 {
 	int b = blockIdx.x;
 	int pl = find_plasma(pre_bucket, P, b);
@@ -1172,13 +1432,15 @@ void k_hist_layout(const Geo *__restrict__ geo, const int *__restrict__ pre_buck
 		return;
 	int tix = tile & (g.ntx - 1), tiy = tile >> g.lgntx;
 	int ox = tix * g.tx - g.M, oy = tiy * g.ty - g.M;
-	int n1 = bucket_n1(bk, b), ntot = n1 + bk.n2[b];
-	for(int j = threadIdx.x; j < ntot; j += blockDim.x)
+	const BucketNow v = bucket_now(bk, par, b);
+	for(int j = threadIdx.x; j < v.n; j += blockDim.x)
 	{
-		int64_t slot = bucket_slot(bk, b, n1, j);
+		int64_t slot = bk.start[b] + j;
 		CellPos c;
-		T rx, ry;
-		locate(g, ox, oy, p_x<T>(p, slot), p_y<T>(p, slot), c, rx, ry);
+		T rx, ry, x = p_x<T>(p, slot);
+		if(!slot_used(v, j, x))
+			continue;
+		locate(g, ox, oy, x, p_y<T>(p, slot), c, rx, ry);
 		int nt = (c.iy >> g.lgty) * g.ntx + (c.ix >> g.lgtx);
 		atomicAdd(&cnt[g.bucket0 + nt * g.ns + s], 1);
 	}
@@ -1281,10 +1543,26 @@ void k_scan_caps(const int *__restrict__ cnt, int nb, double slack, int pad, int
 		*total = big ? -1 : carry;
 }
 
+// Buckets holding cnt[b] particles in their first slots.
+__global__ __launch_bounds__(CPIC_BLOCK)
+void k_bucket_reset(Buckets bk, const int *__restrict__ cnt)
+{
+	int b = blockIdx.x * blockDim.x + threadIdx.x;
+	if(b >= bk.nb)
+		return;
+	const BucketBase v = {cnt[b], 0, 0, 0};
+	const BucketCnt z = {0, 0, 0, 0};
+	for(int par = 0; par < 2; par++)
+	{
+		bk.base[(int64_t) par * bk.nb + b] = v;
+		bk.cnt[(int64_t) par * bk.nb + b] = z;
+	}
+}
+
 template <typename T, bool IDS, bool PE>
 __global__ __launch_bounds__(CPIC_BLOCK)
 void k_scatter_layout(const Geo *__restrict__ geo, const int *__restrict__ pre_bucket, int P,
-		Buckets bk, Parts p, const int *__restrict__ skip, const int64_t *__restrict__ nstart,
+		Buckets bk, int par, Parts p, const int *__restrict__ skip, const int64_t *__restrict__ nstart,
 		int *__restrict__ fill, Parts np)
 {
 	int b = blockIdx.x;
@@ -1296,12 +1574,14 @@ void k_scatter_layout(const Geo *__restrict__ geo, const int *__restrict__ pre_b
 		return;
 	int tix = tile & (g.ntx - 1), tiy = tile >> g.lgntx;
 	int ox = tix * g.tx - g.M, oy = tiy * g.ty - g.M;
-	int n1 = bucket_n1(bk, b), ntot = n1 + bk.n2[b];
-	for(int j = threadIdx.x; j < ntot; j += blockDim.x)
+	const BucketNow v = bucket_now(bk, par, b);
+	for(int j = threadIdx.x; j < v.n; j += blockDim.x)
 	{
-		int64_t slot = bucket_slot(bk, b, n1, j);
+		int64_t slot = bk.start[b] + j;
 		PState<T> q;
 		load_p<T>(p, slot, q, IDS);
+		if(!slot_used(v, j, q.x))
+			continue;
 		if(PE)
 		{
 			q.Ex = p.Ex[slot];
@@ -1362,18 +1642,19 @@ void k_scatter_stage(const Geo *__restrict__ geo, Staged u, const int64_t *__res
 // ------------------------------------------------------------ download ---
 
 __global__ __launch_bounds__(CPIC_BLOCK)
-void k_species_counts(Buckets bk, int bucket0, int ns, int s, int ntiles, int *__restrict__ cnt)
+void k_species_counts(Buckets bk, int par, int bucket0, int ns, int s, int ntiles, int *__restrict__ cnt)
 {
 	for(int t = blockIdx.x * blockDim.x + threadIdx.x; t < ntiles; t += gridDim.x * blockDim.x)
 	{
 		int b = bucket0 + t * ns + s;
-		cnt[t] = bucket_n1(bk, b) + bk.n2[b];
+		BucketNow v = bucket_now(bk, par, b);
+		cnt[t] = v.n - v.holes - (v.gap1 - v.gap0);
 	}
 }
 
 template <typename T, bool IDS, bool PE>
 __global__ __launch_bounds__(CPIC_BLOCK)
-void k_download(Geo g, Buckets bk, Parts p, int s, const int64_t *__restrict__ off,
+void k_download(Geo g, Buckets bk, int par, Parts p, int s, const int64_t *__restrict__ off,
 		double *__restrict__ out /* 6 arrays of n */, int64_t *__restrict__ oid,
 		int64_t *__restrict__ ocell, int64_t n)
 {
@@ -1381,13 +1662,19 @@ void k_download(Geo g, Buckets bk, Parts p, int s, const int64_t *__restrict__ o
 	int b = g.bucket0 + tile * g.ns + s;
 	int tix = tile & (g.ntx - 1), tiy = tile >> g.lgntx;
 	int ox = tix * g.tx - g.M, oy = tiy * g.ty - g.M;
-	int n1 = bucket_n1(bk, b), ntot = n1 + bk.n2[b];
-	for(int j = threadIdx.x; j < ntot; j += blockDim.x)
+	const BucketNow v = bucket_now(bk, par, b);
+	__shared__ int s_done;
+	if(threadIdx.x == 0)
+		s_done = 0;
+	__syncthreads();
+	for(int j = threadIdx.x; j < v.n; j += blockDim.x)
 	{
-		int64_t slot = bucket_slot(bk, b, n1, j);
-		int64_t o = off[tile] + j;
+		int64_t slot = bk.start[b] + j;
 		PState<T> q;
 		load_p<T>(p, slot, q, false);
+		if(!slot_used(v, j, q.x))
+			continue;
+		int64_t o = off[tile] + atomicAdd(&s_done, 1);
 		T x = q.x, y = q.y;
 		CellPos c;
 		T rx, ry;
@@ -1416,19 +1703,21 @@ void k_download(Geo g, Buckets bk, Parts p, int s, const int64_t *__restrict__ o
 
 template <typename T>
 __global__ __launch_bounds__(CPIC_BLOCK)
-void k_cell_counts(Geo g, Buckets bk, Parts p, int s, unsigned long long *__restrict__ counts)
+void k_cell_counts(Geo g, Buckets bk, int par, Parts p, int s, unsigned long long *__restrict__ counts)
 {
 	int tile = blockIdx.x;
 	int b = g.bucket0 + tile * g.ns + s;
 	int tix = tile & (g.ntx - 1), tiy = tile >> g.lgntx;
 	int ox = tix * g.tx - g.M, oy = tiy * g.ty - g.M;
-	int n1 = bucket_n1(bk, b), ntot = n1 + bk.n2[b];
-	for(int j = threadIdx.x; j < ntot; j += blockDim.x)
+	const BucketNow v = bucket_now(bk, par, b);
+	for(int j = threadIdx.x; j < v.n; j += blockDim.x)
 	{
-		int64_t slot = bucket_slot(bk, b, n1, j);
+		int64_t slot = bk.start[b] + j;
 		CellPos c;
-		T rx, ry;
-		locate(g, ox, oy, p_x<T>(p, slot), p_y<T>(p, slot), c, rx, ry);
+		T rx, ry, x = p_x<T>(p, slot);
+		if(!slot_used(v, j, x))
+			continue;
+		locate(g, ox, oy, x, p_y<T>(p, slot), c, rx, ry);
 		atomicAdd(&counts[(int64_t) c.iy * g.nx + c.ix], 1ull);
 	}
 }
@@ -1448,14 +1737,16 @@ void k_cell_counts(Geo g, Buckets bk, Parts p, int s, unsigned long long *__rest
 #define DISPATCH_UU(kern, T, U, EP, ...) do { \
 		bool ids_ = (d->flags & CPIC_F_IDS) != 0; \
 		bool pe_ = (d->flags & CPIC_F_PARTICLE_E) != 0; \
-		if(ids_ && pe_) hipLaunchKernelGGL((kern<T, true, true, U, EP>), __VA_ARGS__); \
-		else if(ids_) hipLaunchKernelGGL((kern<T, true, false, U, EP>), __VA_ARGS__); \
-		else if(pe_) hipLaunchKernelGGL((kern<T, false, true, U, EP>), __VA_ARGS__); \
-		else hipLaunchKernelGGL((kern<T, false, false, U, EP>), __VA_ARGS__); \
+		if(d->bk.compact) hipLaunchKernelGGL((kern<T, false, false, U, EP, true>), __VA_ARGS__); \
+		else if(ids_ && pe_) hipLaunchKernelGGL((kern<T, true, true, U, EP, false>), __VA_ARGS__); \
+		else if(ids_) hipLaunchKernelGGL((kern<T, true, false, U, EP, false>), __VA_ARGS__); \
+		else if(pe_) hipLaunchKernelGGL((kern<T, false, true, U, EP, false>), __VA_ARGS__); \
+		else hipLaunchKernelGGL((kern<T, false, false, U, EP, false>), __VA_ARGS__); \
 	} while(0)
 
 // particles per thread and chunk: 2 (default) or 4, chosen per handle; E
-// from the potential when the E array is stale
+// from the potential when the E array is stale; compact buckets (never with
+// indices or gathered fields)
 #define DISPATCH_U(kern, T, ...) do { \
 		if(d->ppt == 4 && d->E_stale) DISPATCH_UU(kern, T, 4, true, __VA_ARGS__); \
 		else if(d->ppt == 4) DISPATCH_UU(kern, T, 4, false, __VA_ARGS__); \
@@ -1490,12 +1781,14 @@ max_wh(const cpic_dev *d)
 	return m;
 }
 
-// E region plus the rho region, which also holds the potential with its
-// one-node halo while a push computes E from it
+// E region plus the rho region, and the potential with its
+// one-node halo while a push computes E from it: beside them up to 24 KB in all
+// (six workgroups per CU), else in the rho region
+#define PUSH_LDS_APART (24 * 1024)
 size_t
-cpic_push_lds(const cpic_dev *d)
+cpic_push_lds(cpic_dev *d)
 {
-	size_t n = 0, h = 0;
+	size_t n = 0, h = 0, e = d->prec == 64 ? sizeof(double2) : sizeof(float2);
 	for(int p = 0; p < d->P; p++)
 	{
 		size_t w = (size_t) d->hgeo[p].W, hh = (size_t) d->hgeo[p].H;
@@ -1504,7 +1797,9 @@ cpic_push_lds(const cpic_dev *d)
 		if((w + 2) * (hh + 2) > h)
 			h = (w + 2) * (hh + 2);
 	}
-	return n * (d->prec == 64 ? sizeof(double2) : sizeof(float2)) + h * sizeof(double);
+	size_t apart = n * e + (n + h) * sizeof(double);
+	d->phi_apart = apart <= PUSH_LDS_APART;
+	return d->phi_apart ? apart : n * e + h * sizeof(double);
 }
 
 void
@@ -1559,16 +1854,19 @@ push_args(cpic_dev *d, int first, double *rho)
 	a.pre_tile = PRE(d, PRE_TILE);
 	a.pre_bucket = PRE(d, PRE_BUCKET);
 	a.order = d->order;
+	a.units = d->units;
 	a.P = d->P;
 	a.ntiles = d->ntiles;
 	a.bk = d->bk;
 	a.p = d->p[d->pcur];
-	a.q = d->p[1 - d->pcur];
+	a.q = d->p[d->bk.compact ? 1 - d->pcur : d->pcur];
+	a.holes = d->holes;
 	a.lv = d->lv;
-	a.par = d->step_parity;
+	a.par = 1 - d->step_parity;    // of the last push
 	a.first = first;
 	a.E = d->E;
 	a.phi = d->phi;
+	a.phi_apart = d->phi_apart;
 	a.rho = rho;
 	a.diag = (d->flags & CPIC_F_NO_DIAG) ? (DiagSlot *) NULL : d->diag;
 	a.dpart = d->dpart;
@@ -1615,19 +1913,20 @@ cpic_parts_push(cpic_dev *d, int first_iter)
 	PushArgs a = push_args(d, first_iter, d->rho[1 - d->rho_cur]);
 	int slot;
 
-	a.order = d->border;
+	a.par = d->step_parity;
 	slot = cpic_kt_begin(d, "push_gather_deposit");
 	if(d->prec == 64)
-		DISPATCH_U(k_push, double, dim3(d->nb), dim3(PUSH_BLOCK), d->lds_push, d->stream, a);
+		DISPATCH_U(k_push, double, dim3(d->nunits), dim3(PUSH_BLOCK), d->lds_push, d->stream, a);
 	else
-		DISPATCH_U(k_push, float, dim3(d->nb), dim3(PUSH_BLOCK), d->lds_push, d->stream, a);
+		DISPATCH_U(k_push, float, dim3(d->nunits), dim3(PUSH_BLOCK), d->lds_push, d->stream, a);
 	cpic_kt_end(d, slot);
 	HIPCHK(hipGetLastError());
-	d->pcur = 1 - d->pcur;
+	if(d->bk.compact)
+		d->pcur = 1 - d->pcur;
 
 	slot = cpic_kt_begin(d, "append_leavers");
 	DISPATCH_P(k_append, dim3(512), dim3(CPIC_BLOCK), 0, d->stream, d->geo, PRE(d, PRE_BUCKET),
-			d->P, d->bk, d->p[d->pcur], d->lv, d->step_parity, d->ctr, d->st, d->dpart,
+			d->P, d->bk, d->p[d->pcur], d->holes, d->lv, d->step_parity, d->ctr, d->st, d->dpart,
 			(const long long *) a.diag_iter, a.diag, d->ring);
 	cpic_kt_end(d, slot);
 	HIPCHK(hipGetLastError());
@@ -1664,6 +1963,110 @@ cpic_parts_gather(cpic_dev *d)
 	cpic_kt_end(d, slot);
 	HIPCHK(hipGetLastError());
 	return 0;
+}
+
+// Workgroups that share a bucket of n particles, at most `most` each.
+static int
+bucket_parts(int n, int64_t most)
+{
+	int64_t p = ((int64_t) n + most - 1) / most;
+	return (int) (p < 1 ? 1 : p > 0x7fff ? 0x7fff : p);
+}
+
+// The push's work list: every bucket in parts, in XCD bands, so that the parts
+// of one tile run next to each other on one XCD.  A workgroup per bucket
+// leaves much of the chip idle where the buckets are few (256^2 with 32x16
+// tiles: 256 buckets of 16 K particles, one workgroup per CU) and ends late where
+// they differ (ensembles); each part, on the other hand, sets up and
+// flushes the tile's fields again.
+// Buckets of similar sizes take equally many parts, of about 1/1024 of the
+// particles (four workgroups per CU in flight) but not below 2048:
+// FP32 push at 256^2 (4.2 M particles) 59.5 us with 1 part per bucket, 41.2 with
+// 2, 36 with 3-5, 42.4 with 8; at 128^2 (1 M, 128 buckets of 8 K) 33.6 / 23.6 /
+// 19.9 us with 1 / 2 / 4 parts.  FP64 particles (512 a chunk, twice the bytes)
+// gain from 3072 also where buckets are plenty: at 512^2 (16.8 M, 2048
+// buckets of 8 K) 215 / 205 / 202 us with 1 / 2 / 3 parts; FP32 does not
+// (512^2 110 / 113 / 113 us).  Compact buckets are packed by one workgroup each,
+// uneven ones largest first.  Buckets that differ by more than half are cut
+// into parts of at most 6144 (an ensemble of 24 plasmas, 46 M particles: 437 us
+// with 1 part, 322 with 1 part largest first, 332 with parts of 8192 +- half,
+// 297 with at most 6144).  cnt[b] = particles of bucket b (host), or NULL
+// before the first sort.
+#define PUSH_PART_MIN 2048
+#define PUSH_PART_UNEVEN 6144
+#define PUSH_PART_F64 3072
+#define PUSH_PART_UNITS 1024
+static int
+push_units(cpic_dev *d, const int *cnt)
+{
+	const int nb = d->nb;
+	int64_t tot = 0, n = 0;
+	int lo = INT_MAX, hi = 0;
+	for(int b = 0; b < nb; b++)
+	{
+		const int c = cnt ? cnt[b] : 0;
+		tot += c;
+		lo = c < lo ? c : lo;
+		hi = c > hi ? c : hi;
+	}
+	const bool uneven = hi > lo + lo / 2;
+	int64_t target = tot / PUSH_PART_UNITS;
+	if(d->prec == 64 && target > PUSH_PART_F64)
+		target = PUSH_PART_F64;
+	if(target < PUSH_PART_MIN)
+		target = PUSH_PART_MIN;
+	if(d->bk.compact)
+		target = INT_MAX;        // one workgroup packs a bucket
+	else if(uneven)
+	{
+		if(target > PUSH_PART_UNEVEN)
+			target = PUSH_PART_UNEVEN;
+	}
+	else
+	{
+		// as many parts as bring the mean nearest to the target
+		const int64_t mean = tot / nb;
+		int64_t parts = (mean + target / 2) / target;
+		if(parts < 1)
+			parts = 1;
+		target = hi / parts + 1;
+	}
+	for(int b = 0; b < nb; b++)
+		n += bucket_parts(cnt ? cnt[b] : 0, target);
+	if(n > INT_MAX)
+		return CPIC_EINVAL;
+	int2 *u = (int2 *) malloc(sizeof(int2) * 2 * (size_t) n);
+	if(!u)
+		return CPIC_ENOMEM;
+	int64_t k = 0;
+	for(int b = 0; b < nb; b++)
+	{
+		int parts = bucket_parts(cnt ? cnt[b] : 0, target);
+		for(int i = 0; i < parts; i++)
+			u[k++] = make_int2(b, i | parts << 16);
+	}
+	int2 *ord = u + n;
+	for(int64_t i = 0; i < n; i++)
+		ord[i] = u[tile_map((int) i, (int) n)];
+	// whole buckets of uneven sizes: the largest first
+	if(d->bk.compact && uneven)
+		std::stable_sort(ord, ord + n, [cnt](int2 a, int2 b) { return cnt[a.x] > cnt[b.x]; });
+	if(d->unitcap < n)
+	{
+		hipFree(d->units);
+		d->units = NULL;
+		d->unitcap = 0;
+		if(hipMalloc(&d->units, sizeof(int2) * (size_t) n) != hipSuccess)
+		{
+			free(u);
+			return CPIC_ENOMEM;
+		}
+		d->unitcap = (int) n;
+	}
+	hipError_t e = hipMemcpy(d->units, ord, sizeof(int2) * (size_t) n, hipMemcpyHostToDevice);
+	free(u);
+	d->nunits = (int) n;
+	return e == hipSuccess ? 0 : CPIC_EHIP;
 }
 
 // Order in which the tile kernels' blocks take the batch's tiles.  With
@@ -1705,29 +2108,30 @@ cpic_parts_order(cpic_dev *d, const int *cnt)
 	free(ord);
 	if(e != hipSuccess)
 		return CPIC_EHIP;
-	// the same for the buckets (a push by buckets): XCD bands over buckets,
-	// so the buckets of one tile run next to each other on one XCD, largest
-	// first when the counts are uneven
-	const int nb = d->nb;
-	int *bord = (int *) malloc(sizeof(int) * (size_t) nb);
-	if(!bord)
-		return CPIC_ENOMEM;
+	return push_units(d, cnt);
+}
+
+// Whether the push updates the particles in place or packs them into the other
+// buffer: in place while the state fits the memory-side cache (256 MB) a few
+// times; above, the same lines read and written again within microseconds
+// stream slower than one buffer read and another written.  Push times in us, in
+// place / compact: FP32 16.8 M particles (0.27 GB) 127 / 145, 33.6 M (0.54 GB) 238 /
+// 243, 50 M (0.8 GB) 357 / 359, 67 M (1.07 GB) 486 / 467, 134 M (2.1 GB) 974 / 897;
+// FP64 16.8 M (0.54 GB) 194 / 240, 25 M (0.8 GB) 310 / 355, 33.6 M (1.07 GB) 423 /
+// 469, 67 M (2.1 GB) 899 / 892.  Indices and gathered fields stay
+// at their slots, which only the in-place push keeps (packing would move 16 B
+// more per index).
+#define PUSH_INPLACE_F32 0.8e9
+#define PUSH_INPLACE_F64 1.25e9
+static int
+push_in_place(const cpic_dev *d, const int *cnt, int nb)
+{
+	double n = 0;
+	if(d->flags & (CPIC_F_IDS | CPIC_F_PARTICLE_E))
+		return 1;
 	for(int b = 0; b < nb; b++)
-		bord[b] = tile_map(b, nb);
-	if(cnt)
-	{
-		int lo = INT_MAX, hi = 0;
-		for(int b = 0; b < nb; b++)
-		{
-			lo = cnt[b] < lo ? cnt[b] : lo;
-			hi = cnt[b] > hi ? cnt[b] : hi;
-		}
-		if(hi > lo + lo / 2)
-			std::stable_sort(bord, bord + nb, [cnt](int a, int b) { return cnt[a] > cnt[b]; });
-	}
-	e = hipMemcpy(d->border, bord, sizeof(int) * (size_t) nb, hipMemcpyHostToDevice);
-	free(bord);
-	return e == hipSuccess ? 0 : CPIC_EHIP;
+		n += cnt[b];
+	return 4.0 * elem(d) * n <= (d->prec == 64 ? PUSH_INPLACE_F64 : PUSH_INPLACE_F32);
 }
 
 // Full re-sort of the batch: counts per destination bucket (current layout
@@ -1757,6 +2161,7 @@ cpic_parts_rebuild(cpic_dev *d)
 	int *dseg = NULL;
 	int ret = CPIC_ENOMEM, nseg = 0;
 	int touched = 0;         // the particle buffers have been changed
+	const int last = 1 - d->step_parity;   // parity of the last push
 	int *skip = (int *) calloc((size_t) P, sizeof(int));
 	int64_t *segpre = (int64_t *) malloc(sizeof(int64_t) * (size_t) (P * MS + 1));
 	int *seg = (int *) malloc(sizeof(int) * 2 * (size_t) (P * MS));
@@ -1797,10 +2202,10 @@ cpic_parts_rebuild(cpic_dev *d)
 	{
 		if(d->prec == 64)
 			hipLaunchKernelGGL(k_hist_layout<double>, dim3(nb), dim3(CPIC_BLOCK), 0, d->stream,
-					d->geo, PRE(d, PRE_BUCKET), P, d->bk, d->p[d->pcur], dskip, cnt);
+					d->geo, PRE(d, PRE_BUCKET), P, d->bk, last, d->p[d->pcur], dskip, cnt);
 		else
 			hipLaunchKernelGGL(k_hist_layout<float>, dim3(nb), dim3(CPIC_BLOCK), 0, d->stream,
-					d->geo, PRE(d, PRE_BUCKET), P, d->bk, d->p[d->pcur], dskip, cnt);
+					d->geo, PRE(d, PRE_BUCKET), P, d->bk, last, d->p[d->pcur], dskip, cnt);
 	}
 	memset(&u, 0, sizeof(u));
 	if(nseg > 0)
@@ -1870,7 +2275,7 @@ cpic_parts_rebuild(cpic_dev *d)
 				goto out;
 		if(d->pcap[d->pcur] > 0)
 			DISPATCH_P(k_scatter_layout, dim3(nb), dim3(CPIC_BLOCK), 0, d->stream,
-					d->geo, PRE(d, PRE_BUCKET), P, d->bk, d->p[d->pcur], dskip, nstart, fill,
+					d->geo, PRE(d, PRE_BUCKET), P, d->bk, last, d->p[d->pcur], dskip, nstart, fill,
 					d->p[spare]);
 		if(nseg > 0)
 		{
@@ -1880,30 +2285,46 @@ cpic_parts_rebuild(cpic_dev *d)
 					d->geo, u, nstart, fill, d->p[spare]);
 		}
 		RB_CHK(hipGetLastError());
-		// new metadata: n1 = count, res = n2 = 0
+		// new metadata: the counts' slots in use, no holes
 		RB_CHK(hipMemcpyAsync(d->bk.start, nstart, sizeof(int64_t) * nb, hipMemcpyDeviceToDevice, d->stream));
 		RB_CHK(hipMemcpyAsync(d->bk.cap, ncap, sizeof(int) * nb, hipMemcpyDeviceToDevice, d->stream));
-		RB_CHK(hipMemcpyAsync(d->bk.n1, cnt, sizeof(int) * nb, hipMemcpyDeviceToDevice, d->stream));
-		RB_CHK(hipMemsetAsync(d->bk.res, 0, sizeof(int) * nb, d->stream));
-		RB_CHK(hipMemsetAsync(d->bk.n2, 0, sizeof(int) * nb, d->stream));
+		hipLaunchKernelGGL(k_bucket_reset, dim3((nb + CPIC_BLOCK - 1) / CPIC_BLOCK), dim3(CPIC_BLOCK),
+				0, d->stream, d->bk, cnt);
+		RB_CHK(hipGetLastError());
 		RB_CHK(hipStreamSynchronize(d->stream));
 		d->pcur = spare;
-		// the push writes the other buffer: it needs the same capacity
-		if(d->pcap[1 - spare] < d->pcap[spare])
-			if((ret = cpic_parts_alloc(d, 1 - spare, d->pcap[spare])))
-				goto out;
-		// block order for the new counts
+		// the push's buffers and work list for the new counts
 		int *hc = (int *) malloc(sizeof(int) * (size_t) nb);
 		if(!hc)
 		{
 			ret = CPIC_ENOMEM;
 			goto out;
 		}
-		if(hipMemcpy(hc, d->bk.n1, sizeof(int) * nb, hipMemcpyDeviceToHost) != hipSuccess)
+		if(hipMemcpy(hc, cnt, sizeof(int) * nb, hipMemcpyDeviceToHost) != hipSuccess)
 		{
 			free(hc);
 			ret = CPIC_EHIP;
 			goto out;
+		}
+		d->bk.compact = !push_in_place(d, hc, nb);
+		if(d->bk.compact && d->pcap[1 - spare] < d->pcap[spare])
+			if((ret = cpic_parts_alloc(d, 1 - spare, d->pcap[spare])))
+			{
+				free(hc);
+				goto out;
+			}
+		if(!d->bk.compact && d->holecap < d->pcap[spare])
+		{
+			hipFree(d->holes);
+			d->holes = NULL;
+			d->holecap = 0;
+			ret = CPIC_ENOMEM;
+			if(hipMalloc(&d->holes, sizeof(int32_t) * (size_t) d->pcap[spare]) != hipSuccess)
+			{
+				free(hc);
+				goto out;
+			}
+			d->holecap = d->pcap[spare];
 		}
 		ret = cpic_parts_order(d, hc);
 		free(hc);
@@ -1958,7 +2379,7 @@ cpic_parts_download(cpic_dev *d, int plasma, int s, cpic_particles_t *out)
 			hipMalloc(&tot, sizeof(int64_t)) != hipSuccess)
 		goto out;
 	hipLaunchKernelGGL(k_species_counts, dim3((nt + CPIC_BLOCK - 1) / CPIC_BLOCK), dim3(CPIC_BLOCK),
-			0, d->stream, d->bk, g.bucket0, g.ns, s, nt, cnt);
+			0, d->stream, d->bk, 1 - d->step_parity, g.bucket0, g.ns, s, nt, cnt);
 	hipLaunchKernelGGL(k_scan_caps, dim3(1), dim3(1024), 0, d->stream, cnt, nt, 0.0, 0, 1,
 			off, (int *) NULL, tot);
 	HIPCHK(hipMemcpyAsync(&n, tot, sizeof(int64_t), hipMemcpyDeviceToHost, d->stream));
@@ -1976,7 +2397,7 @@ cpic_parts_download(cpic_dev *d, int plasma, int s, cpic_particles_t *out)
 				hipMalloc(&oid, sizeof(int64_t) * n) != hipSuccess ||
 				hipMalloc(&ocell, sizeof(int64_t) * n) != hipSuccess)
 			goto out;
-		DISPATCH_P(k_download, dim3(nt), dim3(CPIC_BLOCK), 0, d->stream, g, d->bk,
+		DISPATCH_P(k_download, dim3(nt), dim3(CPIC_BLOCK), 0, d->stream, g, d->bk, 1 - d->step_parity,
 				d->p[d->pcur], s, off, buf, oid, ocell, n);
 		HIPCHK(hipGetLastError());
 		h = (double *) malloc(sizeof(double) * 6 * n);
@@ -2016,10 +2437,10 @@ cpic_parts_cell_counts(cpic_dev *d, int plasma, int s, int64_t *counts)
 	hipMemsetAsync(c, 0, sizeof(unsigned long long) * n, d->stream);
 	if(d->prec == 64)
 		hipLaunchKernelGGL(k_cell_counts<double>, dim3(g.ntiles), dim3(CPIC_BLOCK), 0, d->stream,
-				g, d->bk, d->p[d->pcur], s, c);
+				g, d->bk, 1 - d->step_parity, d->p[d->pcur], s, c);
 	else
 		hipLaunchKernelGGL(k_cell_counts<float>, dim3(g.ntiles), dim3(CPIC_BLOCK), 0, d->stream,
-				g, d->bk, d->p[d->pcur], s, c);
+				g, d->bk, 1 - d->step_parity, d->p[d->pcur], s, c);
 	hipError_t e = hipMemcpyAsync(counts, c, sizeof(int64_t) * n, hipMemcpyDeviceToHost, d->stream);
 	hipStreamSynchronize(d->stream);
 	hipFree(c);
@@ -2032,22 +2453,46 @@ cpic_parts_init(cpic_dev *d)
 {
 	(void) d;
 	const void *k[] = {
-		(const void *) k_push<double, false, false, 2, false>, (const void *) k_push<double, true, false, 2, false>,
-		(const void *) k_push<double, false, true, 2, false>, (const void *) k_push<double, true, true, 2, false>,
-		(const void *) k_push<float, false, false, 2, false>, (const void *) k_push<float, true, false, 2, false>,
-		(const void *) k_push<float, false, true, 2, false>, (const void *) k_push<float, true, true, 2, false>,
-		(const void *) k_push<double, false, false, 4, false>, (const void *) k_push<double, true, false, 4, false>,
-		(const void *) k_push<double, false, true, 4, false>, (const void *) k_push<double, true, true, 4, false>,
-		(const void *) k_push<float, false, false, 4, false>, (const void *) k_push<float, true, false, 4, false>,
-		(const void *) k_push<float, false, true, 4, false>, (const void *) k_push<float, true, true, 4, false>,
-		(const void *) k_push<double, false, false, 2, true>, (const void *) k_push<double, true, false, 2, true>,
-		(const void *) k_push<double, false, true, 2, true>, (const void *) k_push<double, true, true, 2, true>,
-		(const void *) k_push<float, false, false, 2, true>, (const void *) k_push<float, true, false, 2, true>,
-		(const void *) k_push<float, false, true, 2, true>, (const void *) k_push<float, true, true, 2, true>,
-		(const void *) k_push<double, false, false, 4, true>, (const void *) k_push<double, true, false, 4, true>,
-		(const void *) k_push<double, false, true, 4, true>, (const void *) k_push<double, true, true, 4, true>,
-		(const void *) k_push<float, false, false, 4, true>, (const void *) k_push<float, true, false, 4, true>,
-		(const void *) k_push<float, false, true, 4, true>, (const void *) k_push<float, true, true, 4, true>,
+		(const void *) k_push<double, false, false, 2, false, false>,
+		(const void *) k_push<double, true, false, 2, false, false>,
+		(const void *) k_push<double, false, true, 2, false, false>,
+		(const void *) k_push<double, true, true, 2, false, false>,
+		(const void *) k_push<double, false, false, 2, false, true>,
+		(const void *) k_push<float, false, false, 2, false, false>,
+		(const void *) k_push<float, true, false, 2, false, false>,
+		(const void *) k_push<float, false, true, 2, false, false>,
+		(const void *) k_push<float, true, true, 2, false, false>,
+		(const void *) k_push<float, false, false, 2, false, true>,
+		(const void *) k_push<double, false, false, 2, true, false>,
+		(const void *) k_push<double, true, false, 2, true, false>,
+		(const void *) k_push<double, false, true, 2, true, false>,
+		(const void *) k_push<double, true, true, 2, true, false>,
+		(const void *) k_push<double, false, false, 2, true, true>,
+		(const void *) k_push<float, false, false, 2, true, false>,
+		(const void *) k_push<float, true, false, 2, true, false>,
+		(const void *) k_push<float, false, true, 2, true, false>,
+		(const void *) k_push<float, true, true, 2, true, false>,
+		(const void *) k_push<float, false, false, 2, true, true>,
+		(const void *) k_push<double, false, false, 4, false, false>,
+		(const void *) k_push<double, true, false, 4, false, false>,
+		(const void *) k_push<double, false, true, 4, false, false>,
+		(const void *) k_push<double, true, true, 4, false, false>,
+		(const void *) k_push<double, false, false, 4, false, true>,
+		(const void *) k_push<float, false, false, 4, false, false>,
+		(const void *) k_push<float, true, false, 4, false, false>,
+		(const void *) k_push<float, false, true, 4, false, false>,
+		(const void *) k_push<float, true, true, 4, false, false>,
+		(const void *) k_push<float, false, false, 4, false, true>,
+		(const void *) k_push<double, false, false, 4, true, false>,
+		(const void *) k_push<double, true, false, 4, true, false>,
+		(const void *) k_push<double, false, true, 4, true, false>,
+		(const void *) k_push<double, true, true, 4, true, false>,
+		(const void *) k_push<double, false, false, 4, true, true>,
+		(const void *) k_push<float, false, false, 4, true, false>,
+		(const void *) k_push<float, true, false, 4, true, false>,
+		(const void *) k_push<float, false, true, 4, true, false>,
+		(const void *) k_push<float, true, true, 4, true, false>,
+		(const void *) k_push<float, false, false, 4, true, true>,
 		(const void *) k_deposit<double>, (const void *) k_deposit<float>,
 		(const void *) k_gather<double>, (const void *) k_gather<float>,
 	};
