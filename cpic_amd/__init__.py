@@ -32,7 +32,8 @@ EXPORTS = (
     "cpic_dev_download_field", "cpic_dev_upload_field", "cpic_dev_energy", "cpic_dev_migration",
     "cpic_dev_cell_counts", "cpic_dev_rebuild", "cpic_dev_stats", "cpic_dev_kernel_times",
     "cpic_dev_reset_kernel_times", "cpic_dev_set_profiling", "cpic_batch_create", "cpic_batch_size",
-    "cpic_batch_upload_particles", "cpic_batch_download_particles", "cpic_batch_count",
+    "cpic_batch_upload_particles", "cpic_batch_download_particles",
+    "cpic_batch_download_particles_by_id", "cpic_batch_count",
     "cpic_batch_download_field", "cpic_batch_upload_field", "cpic_batch_energy",
     "cpic_batch_cell_counts", "cpic_adj_create", "cpic_adj_destroy", "cpic_adj_forward",
     "cpic_adj_backward", "cpic_adj_state", "cpic_adj_device_ms", "cpic_adj_set_field_history",
@@ -115,6 +116,7 @@ def lib():
         L.cpic_batch_upload_particles.argtypes = [vp, C.c_int32, C.c_int32, C.c_int64, i64,
                                                   d, d, d, d]
         L.cpic_batch_download_particles.argtypes = [vp, C.c_int32, C.c_int32, P(Particles)]
+        L.cpic_batch_download_particles_by_id.argtypes = [vp, C.c_int32, C.c_int32, P(Particles)]
         L.cpic_batch_count.argtypes = [vp, C.c_int32, C.c_int32, i64]
         L.cpic_batch_download_field.argtypes = [vp, C.c_int32, C.c_int32, d]
         L.cpic_batch_upload_field.argtypes = [vp, C.c_int32, C.c_int32, d]
@@ -232,11 +234,10 @@ class Device:
         p.cell = _ip(out["cell"])
         if "id" in out:
             p.id = _ip(out["id"])
-        check(lib().cpic_batch_download_particles(self._h, plasma, species, C.byref(p)))
+        download = (lib().cpic_batch_download_particles_by_id if sort and "id" in out else
+                    lib().cpic_batch_download_particles)
+        check(download(self._h, plasma, species, C.byref(p)))
         assert p.n == n, (p.n, n)
-        if sort and "id" in out:
-            order = np.argsort(out["id"], kind="stable")
-            out = {k: v[order] for k, v in out.items()}
         return out
 
     def pre_step(self):

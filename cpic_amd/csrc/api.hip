@@ -15,6 +15,7 @@
 // return every pointer to where it was).  The step counter lives on the
 // device, so a replay needs no new kernel arguments.
 #include "dev.h"
+#include "host_sort.h"
 
 #include <cmath>
 #include <stdlib.h>
@@ -170,6 +171,9 @@ dev_free(cpic_dev *d)
 	hipFree(d->lv.src); hipFree(d->lv.count);
 	hipFree(d->diag); hipFree(d->derr); hipFree(d->ctr); hipFree(d->st);
 	hipFree(d->geo); hipFree(d->pre);
+	hipFree(d->dl);
+	if(d->pin)
+		hipHostFree(d->pin);
 	if(d->up_buf)
 		for(int k = 0; k < d->P * CPIC_MAX_SPECIES; k++)
 		{
@@ -515,6 +519,128 @@ cpic_dev_destroy(cpic_dev_t *d)
 	return 0;
 }
 
+// ---------------------------------------------------------- downloads ---
+
+// Copies device ranges to ordinary host memory after the work queued on the
+// handle's stream.  Copying straight into pageable memory runs at ~9 GB/s:
+// the runtime's own staging is one thread's, and for a fresh destination
+// that thread also takes every page fault.  Here the ranges go, DL_CHUNK
+// bytes at a time, through two pinned buffers; while one is filled by DMA,
+// the threads copy the other out, each taking its share of the chunk's pages
+// (and faults).  Small downloads copy on the calling thread: starting threads
+// would cost more than they save.
+int
+cpic_download(cpic_dev *d, int nr, const DlRange *r)
+{
+	struct Piece { size_t at, dst_off, bytes; int range; };
+	std::vector<Piece> pieces;
+	std::vector<size_t> first;         // pieces of chunk c: [first[c], first[c+1])
+	size_t total = 0, fill = DL_CHUNK;
+	if(!d->pin && hipHostMalloc((void **) &d->pin, 2 * DL_CHUNK, hipHostMallocDefault)
+			!= hipSuccess)
+	{
+		d->pin = NULL;
+		return CPIC_ENOMEM;
+	}
+	try
+	{
+		for(int k = 0; k < nr; k++)
+			for(size_t o = 0; o < r[k].bytes; )
+			{
+				if(fill == DL_CHUNK)
+				{
+					first.push_back(pieces.size());
+					fill = 0;
+				}
+				size_t n = std::min(DL_CHUNK - fill, r[k].bytes - o);
+				pieces.push_back({fill, o, n, k});
+				fill += n;
+				o += n;
+				total += n;
+			}
+		first.push_back(pieces.size());
+	}
+	catch(...)
+	{
+		return CPIC_ENOMEM;
+	}
+	const int nchunks = (int) first.size() - 1;
+	const int nt = host_threads((int64_t) total, (int64_t) 1 << 20);
+	std::atomic<int> ready(0), fail(0);
+	std::atomic<int> done[2] = {{0}, {0}};      // shares copied out of each buffer
+	// thread t of n copies its share of every piece of chunk c
+	auto copy_out = [&](int c, int t, int n) {
+		const char *b = d->pin + (size_t) (c & 1) * DL_CHUNK;
+		for(size_t k = first[c]; k < first[c + 1]; k++)
+		{
+			const Piece &p = pieces[k];
+			size_t lo = (p.bytes * (size_t) t / (size_t) n) & ~(size_t) 63;
+			size_t hi = t + 1 == n ? p.bytes :
+				(p.bytes * (size_t) (t + 1) / (size_t) n) & ~(size_t) 63;
+			memcpy((char *) r[p.range].dst + p.dst_off + lo, b + p.at + lo, hi - lo);
+		}
+	};
+	auto fetch = [&](int c) -> hipError_t {
+		char *b = d->pin + (size_t) (c & 1) * DL_CHUNK;
+		for(size_t k = first[c]; k < first[c + 1]; k++)
+		{
+			const Piece &p = pieces[k];
+			hipError_t e = hipMemcpyAsync(b + p.at, (const char *) r[p.range].src + p.dst_off,
+					p.bytes, hipMemcpyDeviceToHost, d->stream);
+			if(e != hipSuccess)
+				return e;
+		}
+		return hipStreamSynchronize(d->stream);
+	};
+	std::vector<std::thread> th;
+	int workers = 0;
+	try
+	{
+		th.reserve((size_t) nt);
+		for(int t = 0; nt > 1 && t < nt; t++)
+		{
+			th.emplace_back([&, t]() {
+				for(int c = 0; c < nchunks; c++)
+				{
+					while(ready.load(std::memory_order_acquire) <= c)
+					{
+						if(fail.load(std::memory_order_relaxed))
+							return;
+						std::this_thread::yield();
+					}
+					copy_out(c, t, nt);
+					done[c & 1].fetch_add(1, std::memory_order_release);
+				}
+			});
+			workers = t + 1;
+		}
+	}
+	catch(...)
+	{
+		// the calling thread copies the other shares
+	}
+	hipError_t e = hipSuccess;
+	for(int c = 0; c < nchunks && e == hipSuccess; c++)
+	{
+		// every share of the buffer's earlier chunks has been copied out
+		while(done[c & 1].load(std::memory_order_acquire) < workers * (c / 2))
+			std::this_thread::yield();
+		if((e = fetch(c)) != hipSuccess)
+			break;
+		ready.store(c + 1, std::memory_order_release);
+		// shares without a thread of their own
+		for(int t = workers; t < nt; t++)
+			copy_out(c, t, nt);
+	}
+	if(e != hipSuccess)
+		fail = 1;
+	for(auto &x : th)
+		x.join();
+	if(e != hipSuccess)
+		fprintf(stderr, "cpic_hip: download failed: %s\n", hipGetErrorString(e));
+	return e == hipSuccess ? 0 : CPIC_EHIP;
+}
+
 // ---------------------------------------------------------- particles ---
 
 static int
@@ -687,8 +813,8 @@ cpic_dev_count(cpic_dev_t *d, int32_t s, int64_t *n)
 	return cpic_batch_count(d, 0, s, n);
 }
 
-extern "C" int
-cpic_batch_download_particles(cpic_dev_t *d, int32_t p, int32_t s, cpic_particles_t *out)
+static int
+download_particles(cpic_dev_t *d, int32_t p, int32_t s, int sorted, cpic_particles_t *out)
 {
 	BROKEN_CHECK(d);
 	int ret;
@@ -701,9 +827,23 @@ cpic_batch_download_particles(cpic_dev_t *d, int32_t p, int32_t s, cpic_particle
 	if((ret = commit(d)))
 		return ret;
 	set_device(d);
-	if((ret = cpic_parts_download(d, p, s, out)))
+	if((ret = cpic_parts_download(d, p, s, sorted, out)))
 		return ret;
 	return derr_check(d);
+}
+
+extern "C" int
+cpic_batch_download_particles(cpic_dev_t *d, int32_t p, int32_t s, cpic_particles_t *out)
+{
+	return download_particles(d, p, s, 0, out);
+}
+
+extern "C" int
+cpic_batch_download_particles_by_id(cpic_dev_t *d, int32_t p, int32_t s, cpic_particles_t *out)
+{
+	if(!d || !(d->flags & CPIC_F_IDS))
+		return CPIC_EINVAL;
+	return download_particles(d, p, s, 1, out);
 }
 
 extern "C" int
@@ -904,8 +1044,9 @@ cpic_dev_step(cpic_dev_t *d, int64_t iter)
 	int ret;
 	if((ret = cpic_dev_field_E(d, iter)))
 		return ret;
-	if((ret = cpic_dev_plasma_E(d, iter)))
-		return ret;
+	// the push stores the E it gathers, so plasma_E's pass of its own is only
+	// for callers that run the stages one by one: 20 us of gather and 5 us
+	// of E array in 72 us per step at 256x64 with 350,017 tracked particles
 	if((ret = cpic_dev_plasma_r(d, iter)))
 		return ret;
 	return cpic_dev_field_rho(d, iter);
@@ -1021,27 +1162,25 @@ cpic_batch_download_field(cpic_dev_t *d, int32_t p, int32_t which, double *out)
 	n = (int64_t) d->hgeo[p].nx * d->hgeo[p].ny;
 	o = d->hgeo[p].node0;
 	set_device(d);
-	if(which == CPIC_RHO)
-		HIPCHK(hipMemcpyAsync(out, d->rho[d->rho_cur] + o, sizeof(double) * n,
-				hipMemcpyDeviceToHost, d->stream));
-	else if(which == CPIC_PHI)
-		HIPCHK(hipMemcpyAsync(out, d->phi + o, sizeof(double) * n, hipMemcpyDeviceToHost,
-				d->stream));
-	else if(which == CPIC_EX || which == CPIC_EY)
+	if(which == CPIC_RHO || which == CPIC_PHI)
+	{
+		const DlRange r = {out, (which == CPIC_RHO ? d->rho[d->rho_cur] : d->phi) + o,
+			sizeof(double) * (size_t) n};
+		return cpic_download(d, 1, &r);
+	}
+	if(which == CPIC_EX || which == CPIC_EY)
 	{
 		int c = which == CPIC_EX ? 0 : 1;
-		int ret = ensure_E(d);
-		if(ret)
+		if((ret = ensure_E(d)))
 			return ret;
 		if(d->prec == 64)
 		{
 			double2 *h = (double2 *) malloc(sizeof(double2) * n);
 			if(!h)
 				return CPIC_ENOMEM;
-			hipMemcpyAsync(h, (double2 *) d->E + o, sizeof(double2) * n, hipMemcpyDeviceToHost,
-					d->stream);
-			hipStreamSynchronize(d->stream);
-			for(int64_t i = 0; i < n; i++)
+			const DlRange r = {h, (double2 *) d->E + o, sizeof(double2) * (size_t) n};
+			ret = cpic_download(d, 1, &r);
+			for(int64_t i = 0; i < n && !ret; i++)
 				out[i] = c ? h[i].y : h[i].x;
 			free(h);
 		}
@@ -1050,18 +1189,16 @@ cpic_batch_download_field(cpic_dev_t *d, int32_t p, int32_t which, double *out)
 			float2 *h = (float2 *) malloc(sizeof(float2) * n);
 			if(!h)
 				return CPIC_ENOMEM;
-			hipMemcpyAsync(h, (float2 *) d->E + o, sizeof(float2) * n, hipMemcpyDeviceToHost,
-					d->stream);
-			hipStreamSynchronize(d->stream);
-			for(int64_t i = 0; i < n; i++)
+			const DlRange r = {h, (float2 *) d->E + o, sizeof(float2) * (size_t) n};
+			ret = cpic_download(d, 1, &r);
+			for(int64_t i = 0; i < n && !ret; i++)
 				out[i] = c ? h[i].y : h[i].x;
 			free(h);
 		}
 	}
 	else
 		return CPIC_EINVAL;
-	HIPCHK(hipStreamSynchronize(d->stream));
-	return 0;
+	return ret;
 }
 
 extern "C" int

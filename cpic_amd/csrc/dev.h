@@ -42,6 +42,8 @@
 #define CPIC_MARGIN 1            // cells of drift covered by the LDS tile regions
 #define CPIC_BUCKET_MAX (1 << 27) // slots of one (tile, species) bucket: 32-bit byte offsets
 #define CPIC_MAX_KERNELS 24
+#define DL_CHUNK ((size_t) 4 << 20)      // bytes of a download's bounce buffer
+#define DL_KEEP ((size_t) 256 << 20)     // largest download workspace a handle keeps
 
 // device error word bits
 #define CPIC_DERR_UMAX 0x1
@@ -142,6 +144,13 @@ struct StepState {
 	long long pad[7];
 };
 
+// One contiguous device range of a download and its host destination.
+struct DlRange {
+	void *dst;
+	const void *src;
+	size_t bytes;
+};
+
 struct KernelTimer {
 	const char *name;
 	int64_t launches;
@@ -232,6 +241,12 @@ struct cpic_dev {
 	int graph_ok;
 	int capturing;           // inside hipStreamBeginCapture/EndCapture
 
+	// downloads: pinned bounce buffers (2 x DL_CHUNK bytes) and the particle
+	// downloads' device workspace, both kept between calls
+	char *pin;
+	char *dl;
+	size_t dlcap;
+
 	// profiling
 	KernelTimer kt[CPIC_MAX_KERNELS];
 	int nkt;
@@ -266,7 +281,8 @@ int cpic_parts_rebuild(cpic_dev *d);
 int cpic_parts_push(cpic_dev *d, int first_iter);
 int cpic_parts_deposit(cpic_dev *d, double *rho_out);
 int cpic_parts_gather(cpic_dev *d);
-int cpic_parts_download(cpic_dev *d, int plasma, int species, cpic_particles_t *out);
+int cpic_parts_download(cpic_dev *d, int plasma, int species, int sorted, cpic_particles_t *out);
+int cpic_download(cpic_dev *d, int n, const DlRange *r);
 int cpic_parts_cell_counts(cpic_dev *d, int plasma, int species, int64_t *counts);
 int cpic_parts_alloc(cpic_dev *d, int which, int64_t cap);
 void cpic_parts_free(cpic_dev *d, int which);

@@ -60,7 +60,7 @@ static void parallel_ranges(int64_t n, int nt, F f)
 // round-robin (one particle of every cell that still has one, per round),
 // so consecutive positions lie in different cells.  Cells are clamped to the
 // grid.  Returns 0, or -1 when memory runs out.
-static int sort_by_cell_rr(int64_t n, const double *x, const double *y, double idx, double idy,
+static inline int sort_by_cell_rr(int64_t n, const double *x, const double *y, double idx, double idy,
 		int nx, int ny, int64_t chunk, int64_t *perm)
 {
 	const int64_t nc = (int64_t) nx * ny;

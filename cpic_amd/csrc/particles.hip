@@ -39,6 +39,7 @@
 // (u_z stays 0).  The translation unit is compiled with -ffp-contract=off;
 // the multiply-adds the reference's clang build contracts are explicit fma().
 #include "dev.h"
+#include "host_sort.h"
 #include "picmath.h"
 
 #include <algorithm>
@@ -1641,9 +1642,23 @@ void k_scatter_stage(const Geo *__restrict__ geo, Staged u, const int64_t *__res
 
 // ------------------------------------------------------------ download ---
 
+// What the host needs to know of a species before its download.
+struct DlInfo {
+	int64_t n;               // particles
+	long long lo, hi;        // smallest and largest index
+	int32_t dup, pad;        // an index met twice
+};
+
 __global__ __launch_bounds__(CPIC_BLOCK)
-void k_species_counts(Buckets bk, int par, int bucket0, int ns, int s, int ntiles, int *__restrict__ cnt)
+void k_species_counts(Buckets bk, int par, int bucket0, int ns, int s, int ntiles,
+		int *__restrict__ cnt, DlInfo *__restrict__ info)
 {
+	if(blockIdx.x == 0 && threadIdx.x == 0)
+	{
+		info->lo = LLONG_MAX;
+		info->hi = LLONG_MIN;
+		info->dup = 0;
+	}
 	for(int t = blockIdx.x * blockDim.x + threadIdx.x; t < ntiles; t += gridDim.x * blockDim.x)
 	{
 		int b = bucket0 + t * ns + s;
@@ -1652,17 +1667,51 @@ void k_species_counts(Buckets bk, int par, int bucket0, int ns, int s, int ntile
 	}
 }
 
+// Range of the indices of species s, one block per tile.
+template <typename T>
+__global__ __launch_bounds__(CPIC_BLOCK)
+void k_id_range(Geo g, Buckets bk, int par, Parts p, int s, DlInfo *__restrict__ info)
+{
+	const int b = g.bucket0 + blockIdx.x * g.ns + s;
+	const BucketNow v = bucket_now(bk, par, b);
+	long long lo = LLONG_MAX, hi = LLONG_MIN;
+	for(int j = threadIdx.x; j < v.n; j += blockDim.x)
+	{
+		int64_t slot = bk.start[b] + j;
+		if(!slot_used(v, j, p_x<T>(p, slot)))
+			continue;
+		long long id = p.id[slot];
+		lo = min(lo, id);
+		hi = max(hi, id);
+	}
+	for(int off = 32; off > 0; off >>= 1)
+	{
+		lo = min(lo, (long long) __shfl_xor(lo, off));
+		hi = max(hi, (long long) __shfl_xor(hi, off));
+	}
+	if((threadIdx.x & 63) == 0 && lo <= hi)
+	{
+		atomicMin(&info->lo, lo);
+		atomicMax(&info->hi, hi);
+	}
+}
+
+// The species as arrays (x, y, ux, uy, Ex, Ey, index, cell, n elements each):
+// in storage order, or with `seen` (n bits, zero) particle i at position
+// i - info->lo, which the caller has found to be below n for all of them.
 template <typename T, bool IDS, bool PE>
 __global__ __launch_bounds__(CPIC_BLOCK)
 void k_download(Geo g, Buckets bk, int par, Parts p, int s, const int64_t *__restrict__ off,
-		double *__restrict__ out /* 6 arrays of n */, int64_t *__restrict__ oid,
-		int64_t *__restrict__ ocell, int64_t n)
+		double *__restrict__ out, int64_t n, DlInfo *__restrict__ info,
+		unsigned *__restrict__ seen)
 {
 	int tile = blockIdx.x;
 	int b = g.bucket0 + tile * g.ns + s;
 	int tix = tile & (g.ntx - 1), tiy = tile >> g.lgntx;
 	int ox = tix * g.tx - g.M, oy = tiy * g.ty - g.M;
 	const BucketNow v = bucket_now(bk, par, b);
+	int64_t *__restrict__ oid = (int64_t *) (out + 6 * n), *__restrict__ ocell = oid + n;
+	const long long lo = seen ? info->lo : 0;
 	__shared__ int s_done;
 	if(threadIdx.x == 0)
 		s_done = 0;
@@ -1671,10 +1720,21 @@ void k_download(Geo g, Buckets bk, int par, Parts p, int s, const int64_t *__res
 	{
 		int64_t slot = bk.start[b] + j;
 		PState<T> q;
-		load_p<T>(p, slot, q, false);
+		load_p<T>(p, slot, q, IDS);
 		if(!slot_used(v, j, q.x))
 			continue;
-		int64_t o = off[tile] + atomicAdd(&s_done, 1);
+		int64_t o;
+		if(IDS && seen)
+		{
+			o = q.id - lo;
+			unsigned bit = 1u << (o & 31);
+			if(o >= 0 && o < n && (atomicOr(&seen[o >> 5], bit) & bit))
+				info->dup = 1;
+		}
+		else
+			o = off[tile] + atomicAdd(&s_done, 1);
+		if(o < 0 || o >= n)
+			continue;
 		T x = q.x, y = q.y;
 		CellPos c;
 		T rx, ry;
@@ -1694,9 +1754,13 @@ void k_download(Geo g, Buckets bk, int par, Parts p, int s, const int64_t *__res
 		out[n + o] = ay;
 		out[2 * n + o] = (double) q.ux;
 		out[3 * n + o] = (double) q.uy;
-		out[4 * n + o] = PE ? p.Ex[slot] : 0.0;
-		out[5 * n + o] = PE ? p.Ey[slot] : 0.0;
-		oid[o] = IDS ? p.id[slot] : -1;
+		if(PE)
+		{
+			out[4 * n + o] = p.Ex[slot];
+			out[5 * n + o] = p.Ey[slot];
+		}
+		if(IDS)
+			oid[o] = q.id;
 		ocell[o] = (int64_t) c.iy * g.nx + c.ix;
 	}
 }
@@ -2361,69 +2425,141 @@ out:
 	return ret;
 }
 
+// One species as host arrays, in storage order or sorted by index (equal
+// indices in storage order).  When the species' indices are the consecutive
+// ones lo .. lo + n - 1, as a program that numbers its particles has them, each
+// particle's index is its position: the kernel writes the arrays in order (a
+// bit per index finds one that occurs twice).  Any other set is sorted on the
+// host.  Only the arrays asked for are copied.
+// 256x64, three species of 350,017 particles, index and gathered E: a pass of
+// 20 steps and all downloads 31.0 ms with unordered downloads that the caller
+// sorts, 3.31 ms so (2 x 5,120 particles at 64^2, 100 steps: 3.91 -> 3.53 ms).
 int
-cpic_parts_download(cpic_dev *d, int plasma, int s, cpic_particles_t *out)
+cpic_parts_download(cpic_dev *d, int plasma, int s, int sorted, cpic_particles_t *out)
 {
 	const Geo &g = d->hgeo[plasma];
-	int nt = g.ntiles;
-	int *cnt = NULL;
-	int64_t *off = NULL, *tot = NULL, n = 0;
-	double *buf = NULL;
-	int64_t *oid = NULL, *ocell = NULL;
-	double *h = NULL;
-	int64_t *hid = NULL, *hcell = NULL;
-	int ret = CPIC_ENOMEM;
+	const int nt = g.ntiles, par = 1 - d->step_parity;
+	// every particle is in a bucket, so the counts' sum is the upload's
+	const int64_t n = d->count[plasma * CPIC_MAX_SPECIES + s];
+	void *const dst[8] = {out->x, out->y, out->ux, out->uy, out->Ex, out->Ey, out->id, out->cell};
+	DlInfo info;
+	int ret, arrays = 0;
 
-	if(hipMalloc(&cnt, sizeof(int) * nt) != hipSuccess ||
-			hipMalloc(&off, sizeof(int64_t) * nt) != hipSuccess ||
-			hipMalloc(&tot, sizeof(int64_t)) != hipSuccess)
-		goto out;
-	hipLaunchKernelGGL(k_species_counts, dim3((nt + CPIC_BLOCK - 1) / CPIC_BLOCK), dim3(CPIC_BLOCK),
-			0, d->stream, d->bk, 1 - d->step_parity, g.bucket0, g.ns, s, nt, cnt);
-	hipLaunchKernelGGL(k_scan_caps, dim3(1), dim3(1024), 0, d->stream, cnt, nt, 0.0, 0, 1,
-			off, (int *) NULL, tot);
-	HIPCHK(hipMemcpyAsync(&n, tot, sizeof(int64_t), hipMemcpyDeviceToHost, d->stream));
-	HIPCHK(hipStreamSynchronize(d->stream));
-	if(out->n < n && (out->x || out->y || out->ux || out->uy || out->id || out->Ex ||
-				out->Ey || out->cell))
+	for(int k = 0; k < 8; k++)
+		arrays += dst[k] != NULL;
+	if(out->n < n && arrays)
 	{
 		out->n = n;
-		ret = CPIC_EINVAL;
-		goto out;
-	}
-	if(n > 0)
-	{
-		if(hipMalloc(&buf, sizeof(double) * 6 * n) != hipSuccess ||
-				hipMalloc(&oid, sizeof(int64_t) * n) != hipSuccess ||
-				hipMalloc(&ocell, sizeof(int64_t) * n) != hipSuccess)
-			goto out;
-		DISPATCH_P(k_download, dim3(nt), dim3(CPIC_BLOCK), 0, d->stream, g, d->bk, 1 - d->step_parity,
-				d->p[d->pcur], s, off, buf, oid, ocell, n);
-		HIPCHK(hipGetLastError());
-		h = (double *) malloc(sizeof(double) * 6 * n);
-		hid = (int64_t *) malloc(sizeof(int64_t) * n);
-		hcell = (int64_t *) malloc(sizeof(int64_t) * n);
-		if(!h || !hid || !hcell)
-			goto out;
-		HIPCHK(hipMemcpyAsync(h, buf, sizeof(double) * 6 * n, hipMemcpyDeviceToHost, d->stream));
-		HIPCHK(hipMemcpyAsync(hid, oid, sizeof(int64_t) * n, hipMemcpyDeviceToHost, d->stream));
-		HIPCHK(hipMemcpyAsync(hcell, ocell, sizeof(int64_t) * n, hipMemcpyDeviceToHost, d->stream));
-		HIPCHK(hipStreamSynchronize(d->stream));
-		if(out->x) memcpy(out->x, h, sizeof(double) * n);
-		if(out->y) memcpy(out->y, h + n, sizeof(double) * n);
-		if(out->ux) memcpy(out->ux, h + 2 * n, sizeof(double) * n);
-		if(out->uy) memcpy(out->uy, h + 3 * n, sizeof(double) * n);
-		if(out->Ex) memcpy(out->Ex, h + 4 * n, sizeof(double) * n);
-		if(out->Ey) memcpy(out->Ey, h + 5 * n, sizeof(double) * n);
-		if(out->id) memcpy(out->id, hid, sizeof(int64_t) * n);
-		if(out->cell) memcpy(out->cell, hcell, sizeof(int64_t) * n);
+		return CPIC_EINVAL;
 	}
 	out->n = n;
-	ret = 0;
-out:
-	hipFree(cnt); hipFree(off); hipFree(tot); hipFree(buf); hipFree(oid); hipFree(ocell);
-	free(h); free(hid); free(hcell);
-	return ret;
+	if(n == 0 || !arrays)
+		return 0;
+
+	// workspace: info, tile offsets and counts, the arrays, a bit per index
+	const size_t o_off = 256, o_cnt = o_off + sizeof(int64_t) * (size_t) nt;
+	const size_t o_out = (o_cnt + sizeof(int) * (size_t) nt + 255) & ~(size_t) 255;
+	const size_t o_seen = o_out + 8 * sizeof(double) * (size_t) n;
+	const int64_t words = (n + 63) / 64;
+	const size_t need = o_seen + (size_t) words * 8;
+	if(d->dlcap < need)
+	{
+		hipFree(d->dl);
+		d->dl = NULL;
+		d->dlcap = 0;
+		if(hipMalloc((void **) &d->dl, need) != hipSuccess)
+		{
+			d->dl = NULL;
+			(void) hipGetLastError();
+			return CPIC_ENOMEM;
+		}
+		d->dlcap = need;
+	}
+	DlInfo *dinfo = (DlInfo *) d->dl;
+	int64_t *off = (int64_t *) (d->dl + o_off);
+	int *cnt = (int *) (d->dl + o_cnt);
+	double *buf = (double *) (d->dl + o_out);
+	unsigned *seen = (unsigned *) (d->dl + o_seen);
+	const DlRange rinfo = {&info, dinfo, sizeof(info)};
+	const dim3 grid(nt), block(CPIC_BLOCK);
+
+	hipLaunchKernelGGL(k_species_counts, dim3((nt + CPIC_BLOCK - 1) / CPIC_BLOCK), block,
+			0, d->stream, d->bk, par, g.bucket0, g.ns, s, nt, cnt, dinfo);
+	bool dense = false;
+	if(sorted)
+	{
+		if(d->prec == 64)
+			hipLaunchKernelGGL(k_id_range<double>, grid, block, 0, d->stream, g, d->bk, par,
+					d->p[d->pcur], s, dinfo);
+		else
+			hipLaunchKernelGGL(k_id_range<float>, grid, block, 0, d->stream, g, d->bk, par,
+					d->p[d->pcur], s, dinfo);
+		HIPCHK(hipGetLastError());
+		if((ret = cpic_zero(d, (double *) seen, words)) || (ret = cpic_download(d, 1, &rinfo)))
+			return ret;
+		dense = (uint64_t) info.hi - (uint64_t) info.lo == (uint64_t) n - 1;
+	}
+	int64_t *order = NULL;
+	for(;;)
+	{
+		if(!dense)
+			hipLaunchKernelGGL(k_scan_caps, dim3(1), dim3(1024), 0, d->stream, cnt, nt, 0.0, 0, 1,
+					off, (int *) NULL, &dinfo->n);
+		DISPATCH_P(k_download, grid, block, 0, d->stream, g, d->bk, par, d->p[d->pcur], s, off,
+				buf, n, dinfo, dense ? seen : (unsigned *) NULL);
+		HIPCHK(hipGetLastError());
+		DlRange r[9];
+		int nr = 0;
+		for(int k = 0; k < 8; k++)
+			if(dst[k])
+				r[nr++] = {dst[k], buf + (int64_t) k * n, sizeof(double) * (size_t) n};
+		int64_t *ids = NULL;
+		if(sorted && !dense)
+		{
+			ids = (int64_t *) malloc(2 * sizeof(int64_t) * (size_t) n);
+			if(!ids)
+				return CPIC_ENOMEM;
+			r[nr++] = {ids, buf + 6 * n, sizeof(int64_t) * (size_t) n};
+		}
+		else if(sorted)
+			r[nr++] = rinfo;
+		if((ret = cpic_download(d, nr, r)))
+		{
+			free(ids);
+			return ret;
+		}
+		if(ids)
+		{
+			order = ids + n;
+			for(int64_t i = 0; i < n; i++)
+				order[i] = i;
+			std::stable_sort(order, order + n, [&](int64_t a, int64_t b) { return ids[a] < ids[b]; });
+			int64_t *tmp = (int64_t *) malloc(sizeof(int64_t) * (size_t) n);
+			if(!tmp)
+			{
+				free(ids);
+				return CPIC_ENOMEM;
+			}
+			for(int k = 0; k < 8; k++)
+				if(dst[k])
+				{
+					memcpy(tmp, dst[k], sizeof(int64_t) * (size_t) n);
+					gather_perm(n, order, (const int64_t *) tmp, (int64_t *) dst[k]);
+				}
+			free(tmp);
+			free(ids);
+		}
+		if(!dense || !info.dup)
+			break;
+		dense = false;
+	}
+	if(d->dlcap > DL_KEEP)
+	{
+		hipFree(d->dl);
+		d->dl = NULL;
+		d->dlcap = 0;
+	}
+	return 0;
 }
 
 int

@@ -242,6 +242,10 @@ int cpic_batch_upload_particles(cpic_dev_t *dev, int32_t plasma, int32_t species
 		const double *ux, const double *uy);
 int cpic_batch_download_particles(cpic_dev_t *dev, int32_t plasma, int32_t species,
 		cpic_particles_t *out);
+/* The same sorted by particle index, equal indices in storage order; needs
+ * CPIC_F_IDS (the id array itself may be NULL). */
+int cpic_batch_download_particles_by_id(cpic_dev_t *dev, int32_t plasma, int32_t species,
+		cpic_particles_t *out);
 int cpic_batch_count(cpic_dev_t *dev, int32_t plasma, int32_t species, int64_t *n);
 int cpic_batch_download_field(cpic_dev_t *dev, int32_t plasma, int32_t which, double *out);
 int cpic_batch_upload_field(cpic_dev_t *dev, int32_t plasma, int32_t which,
