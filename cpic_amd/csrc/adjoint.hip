@@ -18,10 +18,11 @@
 //   lrho = S psi                       (S is symmetric: real, even G)
 //   lr = lr' + grad Gat(E)(r) . lE_p + c grad Gat(lrho)(r),  c = -q/e0
 // (the last two are derivatives of the CIC interpolant with respect to the
-// particle position).  States are checkpointed every K iterations in the
-// forward, which also keeps every iteration's rho and E when they fit a
-// fixed budget; the reverse recomputes each segment's positions from its
-// checkpoint (and, without that history, their rho and E).  No counterpart
+// particle position).  The forward keeps every iteration's rho, E and
+// positions when they fit fixed budgets, and the reverse reads them.  Otherwise
+// states are checkpointed every K iterations and the reverse recomputes each
+// segment's positions from its checkpoint (and, without the field history,
+// their rho and E).  No counterpart
 // in the reference, which has no gradients.
 #include "dev.h"
 #include "host_sort.h"
@@ -66,6 +67,12 @@ struct cpic_adj {
 	double *frho, *fE;
 	int64_t frhocap, fEcap;   // doubles
 	int fhist;                // the last forward kept it
+	// position history of the last forward (with the field history, when it
+	// fits ADJ_POS_HISTORY_MAX and is not switched off): x, then y of
+	// iterations 0..T-1, which leaves the reverse sweep nothing to recompute
+	double *ph;
+	int64_t phcap;
+	int phist, phist_off;
 	int fhist_off;            // cpic_adj_set_field_history(a, 0)
 	double *wk;               // recompute state of the reverse sweep, 4n doubles
 	hipEvent_t ev[4];         // device work of the last forward [0,1] and backward [2,3]
@@ -416,6 +423,14 @@ static_assert(ADJ_CHUNK % REV_CHUNK == 0, "reverse blocks split the sort's chunk
 // iteration, 24 B per node and iteration: 315 MB for 200 iterations at
 // 256^2); beyond it the reverse sweep recomputes each segment's fields
 #define ADJ_FIELD_HISTORY_MAX ((int64_t) 8 << 30)
+// Device memory the position history may take (16 B per particle and
+// iteration: 13.4 GB for 200 iterations of 4,194,304 particles), and at most
+// half of what is free.  The forward's push writes each iteration's positions
+// there instead of in place, at no extra traffic, and the reverse sweep reads
+// them instead of pushing every segment's particles again from a
+// checkpoint: 4,194,304 particles, 200 steps, forward and backward 78.4 -> 69.8 ms (11 ms of recompute);
+// the checkpoints (134 MB of copies each there) are not taken either.
+#define ADJ_POS_HISTORY_MAX ((int64_t) 32 << 30)
 template <bool PEND>
 __global__ __launch_bounds__(CPIC_BLOCK)
 void k_adj_rev_a(Geo g, AdjSpecies k, int set_r, double dtp, int64_t n,
@@ -573,7 +588,7 @@ adj_free(cpic_adj *a)
 	hipFree(a->E); hipFree(a->lE);
 	hipFree(a->lx); hipFree(a->ly); hipFree(a->lux); hipFree(a->luy);
 	hipFree(a->ck); hipFree(a->seg); hipFree(a->segf); hipFree(a->hist);
-	hipFree(a->frho); hipFree(a->fE);
+	hipFree(a->frho); hipFree(a->fE); hipFree(a->ph);
 	hipFree(a->derr);
 	hipFree(a->wk);
 	if(a->evok)
@@ -836,6 +851,28 @@ download_unsorted(cpic_adj *a, double *const *src, double *const *dst)
 	return 0;
 }
 
+// Whether this forward keeps its position history, whose memory is then there.
+static bool
+pos_history(cpic_adj *a, int64_t nsteps)
+{
+	size_t avail = 0, total = 0;
+	double want = 2.0 * (double) a->n * (double) nsteps;
+	if(a->phist_off || want * sizeof(double) > (double) ADJ_POS_HISTORY_MAX)
+		return false;
+	if((double) a->phcap >= want)
+		return true;
+	if(hipMemGetInfo(&avail, &total) != hipSuccess ||
+			want * sizeof(double) > 0.5 * ((double) avail + 8.0 * (double) a->phcap))
+	{
+		(void) hipGetLastError();
+		return false;
+	}
+	if(!grow(&a->ph, &a->phcap, (int64_t) want))
+		return true;
+	(void) hipGetLastError();   // no room: checkpoints instead
+	return false;
+}
+
 extern "C" int
 cpic_adj_forward(cpic_adj_t *a, const double *x, const double *y, const double *ux,
 		const double *uy, int64_t nsteps, int32_t checkpoint_every, double *loss,
@@ -858,7 +895,7 @@ cpic_adj_forward(cpic_adj_t *a, const double *x, const double *y, const double *
 		return CPIC_EINVAL;
 	hipSetDevice(a->d->device);
 	int64_t K = checkpoint_every, nck = (nsteps + K - 1) / K, n = a->n;
-	if((ret = grow(&a->ck, &a->ckcap, 4 * n * nck)) || (ret = grow(&a->hist, &a->histcap, nsteps)))
+	if((ret = grow(&a->hist, &a->histcap, nsteps)))
 		return ret;
 	if((ret = sort_by_cell(a, x, y)))
 		return ret;
@@ -897,19 +934,34 @@ cpic_adj_forward(cpic_adj_t *a, const double *x, const double *y, const double *
 		else
 			(void) hipGetLastError();   // no room: the reverse recomputes instead
 	}
+	a->phist = a->fhist && pos_history(a, nsteps);
+	if(!a->phist && (ret = grow(&a->ck, &a->ckcap, 4 * n * nck)))
+		return ret;
 	HIPCHK(hipEventRecord(a->ev[0], a->d->stream));
 	if((ret = deposit(a, a->x, a->y, a->fhist ? a->frho : a->rho[0])) ||
 			(ret = zero(a, a->hist, nsteps)))
 		return ret;
 	for(int64_t it = 0; it < nsteps; it++)
 	{
-		if(it % K == 0)
+		if(a->phist && it == 0)
+		{
+			if((ret = copy_state(a, a->ph, a->x, a->y, NULL, NULL, hipMemcpyDeviceToDevice)))
+				return ret;
+		}
+		else if(!a->phist && it % K == 0)
 			if((ret = copy_state(a, a->ck + 4 * n * (it / K), a->x, a->y, a->ux, a->uy,
 					hipMemcpyDeviceToDevice)))
 				return ret;
 		if(a->fhist)
-			ret = forward_step(a, it, a->x, a->y, a->x, a->y, a->frho + nodes * it,
+		{
+			// with the position history, from its slot to the next one or, the
+			// last, to the state
+			double *from = a->phist ? a->ph + 2 * n * it : NULL;
+			bool last = !a->phist || it + 1 == nsteps;
+			ret = forward_step(a, it, from ? from : a->x, from ? from + n : a->y,
+					last ? a->x : from + 2 * n, last ? a->y : from + 3 * n, a->frho + nodes * it,
 					a->frho + nodes * (it + 1), (double2 *) a->fE + nodes * it, a->hist + it);
+		}
 		else
 			ret = forward_iter(a, it, &cur, a->hist + it);
 		if(ret)
@@ -970,6 +1022,15 @@ cpic_adj_set_field_history(cpic_adj_t *a, int on)
 }
 
 extern "C" int
+cpic_adj_set_position_history(cpic_adj_t *a, int on)
+{
+	if(!a)
+		return CPIC_EINVAL;
+	a->phist_off = !on;
+	return 0;
+}
+
+extern "C" int
 cpic_adj_state(cpic_adj_t *a, double *x, double *y, double *ux, double *uy)
 {
 	if(!a || !a->have)
@@ -988,13 +1049,14 @@ cpic_adj_backward(cpic_adj_t *a, double dloss, double *gx, double *gy, double *g
 	if(!a || !a->have)
 		return CPIC_EINVAL;
 	hipSetDevice(a->d->device);
-	const int64_t n = a->n, K = a->K, T = a->nsteps, nodes = (int64_t) a->g.nx * a->g.ny;
-	const int64_t nck = (T + K - 1) / K;
+	const int64_t n = a->n, T = a->nsteps, K = a->phist ? T : a->K, nodes = (int64_t) a->g.nx * a->g.ny;
+	const int fh = a->fhist, ph = a->phist;
+	// with the position history one segment is the whole run
+	const int64_t nck = ph ? 1 : (T + K - 1) / K;
 	// a segment holds at most min(K, T) iterations (the last one T - (nck-1) K),
 	// the positions of all but its first in the segment buffer
 	const int64_t Kseg = K < T ? K : T;
-	const int fh = a->fhist;
-	if((ret = grow(&a->seg, &a->segcap, 2 * n * (Kseg - 1))) ||
+	if((!ph && (ret = grow(&a->seg, &a->segcap, 2 * n * (Kseg - 1)))) ||
 			(!fh && (ret = grow(&a->segf, &a->segfcap, 3 * nodes * Kseg))))
 		return ret;
 	if(!a->wk && hipMalloc(&a->wk, sizeof(double) * 4 * (size_t) n) != hipSuccess)
@@ -1035,11 +1097,13 @@ cpic_adj_backward(cpic_adj_t *a, double dloss, double *gx, double *gy, double *g
 		// positions (x, then y) of iteration it: the checkpoint's for the
 		// segment's first, slot it - it0 - 1 of the segment buffer, which the
 		// recompute's pushes write, for the others
-		const double *c = a->ck + 4 * n * sg;
+		const double *c = ph ? a->ph : a->ck + 4 * n * sg;
 		auto slot = [&](int64_t it) -> double * { return a->seg + 2 * n * (it - it0 - 1); };
-		auto pos = [&](int64_t it) -> const double * { return it == it0 ? c : slot(it); };
+		auto pos = [&](int64_t it) -> const double * {
+			return ph ? a->ph + 2 * n * it : it == it0 ? c : slot(it);
+		};
 		// velocities only for a segment that moves its particles
-		if(it1 - it0 > 1 &&
+		if(!ph && it1 - it0 > 1 &&
 				(hipMemcpyAsync(a->ux, c + 2 * n, sizeof(double) * n, hipMemcpyDeviceToDevice,
 						a->d->stream) != hipSuccess ||
 				hipMemcpyAsync(a->uy, c + 3 * n, sizeof(double) * n, hipMemcpyDeviceToDevice,
@@ -1048,7 +1112,9 @@ cpic_adj_backward(cpic_adj_t *a, double dloss, double *gx, double *gy, double *g
 			ret = CPIC_EHIP;
 			break;
 		}
-		if(fh)
+		if(ph)
+			;                  // positions and fields are there
+		else if(fh)
 		{
 			// positions only, moved by the history's E
 			for(int64_t it = it0; it + 1 < it1 && !ret; it++)
@@ -1104,11 +1170,13 @@ cpic_adj_backward(cpic_adj_t *a, double dloss, double *gx, double *gy, double *g
 				break;
 		}
 	}
-	// the lrho term of iteration 0 (positions: the first checkpoint's)
+	// the lrho term of iteration 0 (its positions: the history's or the first
+	// checkpoint's)
+	const double *r0 = ph ? a->ph : a->ck;
 	if(!ret)
 	{
 		hipLaunchKernelGGL(k_adj_rev_b, dim3(pblocks(n)), dim3(CPIC_BLOCK), 0, a->d->stream,
-				a->g, a->k[1], n, a->sp, (const double *) a->ck, (const double *) a->ck + n,
+				a->g, a->k[1], n, a->sp, r0, r0 + n,
 				(const double *) a->lrho, a->lx, a->ly);
 		if(hipGetLastError() != hipSuccess)
 			ret = CPIC_EHIP;

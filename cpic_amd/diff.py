@@ -70,6 +70,11 @@ class AdjointRun:
         fit) for the backward, instead of its recomputing them."""
         ca.check(ca.lib().cpic_adj_set_field_history(self._h, 1 if on else 0))
 
+    def set_position_history(self, on):
+        """Whether later forwards keep every iteration's positions with the
+        fields (when they fit) instead of checkpoints."""
+        ca.check(ca.lib().cpic_adj_set_position_history(self._h, 1 if on else 0))
+
     def device_ms(self):
         """Device time of the last forward and backward in ms (-1 if not run)."""
         f, b = C.c_double(), C.c_double()

@@ -261,12 +261,15 @@ int cpic_batch_cell_counts(cpic_dev_t *dev, int32_t plasma, int32_t species,
  * that keep their index, and return reverse-mode gradients of the
  * time-integrated field energy  loss = sum_{it < nsteps} W(it),
  * W = -(e0/2) sum rho*phi  (the value cpic_dev_energy reports per step),
- * with respect to every particle's initial position and velocity.  Forward
- * states are checkpointed every `checkpoint_every` iterations and the
- * reverse sweep recomputes each segment's positions from its checkpoint;
- * the fields of every iteration (rho and E, 24 bytes per node and
- * iteration) are kept by the forward when they fit 8 GiB of device memory
- * (cpic_adj_set_field_history), else recomputed with the positions.  desc
+ * with respect to every particle's initial position and velocity.  The
+ * forward keeps the fields of every iteration (rho and E, 24 bytes per node
+ * and iteration) when they fit 8 GiB of device memory
+ * (cpic_adj_set_field_history) and with them every iteration's positions (16
+ * bytes per particle and iteration) when they fit 32 GiB and half of the free
+ * memory (cpic_adj_set_position_history).  Without the positions, states are
+ * checkpointed every `checkpoint_every` iterations and the reverse sweep
+ * recomputes each segment's positions from its checkpoint, and without the
+ * fields those too.  desc
  * must have precision 64; flags, tile and slack are ignored.
  */
 typedef struct cpic_adj cpic_adj_t;
@@ -303,6 +306,11 @@ int cpic_adj_device_ms(cpic_adj_t *adj, double *forward_ms, double *backward_ms)
  * what its forward did.  No counterpart in the reference, which has no
  * differentiable run. */
 int cpic_adj_set_field_history(cpic_adj_t *adj, int on);
+
+/* The same for the positions: on = 0 makes later forwards checkpoint every
+ * `checkpoint_every` iterations instead (less memory); on = 1 (the default):
+ * keep them with the fields when they fit. */
+int cpic_adj_set_position_history(cpic_adj_t *adj, int on);
 
 #ifdef __cplusplus
 }
