@@ -25,7 +25,6 @@
 // their rho and E).  No counterpart
 // in the reference, which has no gradients.
 #include "dev.h"
-#include "host_sort.h"
 #include "picmath.h"
 
 #include <cmath>
@@ -45,10 +44,9 @@ struct cpic_adj {
 	int64_t n;
 	int ns;
 	AdjSpecies k[2];          // [0]: iteration 0 (dt' = -dt/2), [1]: later iterations
-	int32_t *sp;              // species of each particle (device, in sorted order)
-	int32_t *hsp;             // species of each particle (host, caller's order)
+	uint8_t *sp;              // species of each particle, in sorted order
+	uint8_t *sp0;             // the same in the caller's order
 	int64_t *perm;            // sorted position i holds the caller's particle perm[i]
-	double *hbuf;             // host staging, 4n doubles (pinned)
 	double *x, *y, *ux, *uy;  // state
 	double *rho[2], *phi, *psi, *lrho;
 	double2 *E, *lE;          // lE: two buffers of nodes values (reverse iterations alternate)
@@ -74,7 +72,8 @@ struct cpic_adj {
 	int64_t phcap;
 	int phist, phist_off;
 	int fhist_off;            // cpic_adj_set_field_history(a, 0)
-	double *wk;               // recompute state of the reverse sweep, 4n doubles
+	double *wk;               // recompute state of the reverse sweep, and x, y, ux, uy in
+	                          // the caller's order on their way in and out: 4n doubles
 	hipEvent_t ev[4];         // device work of the last forward [0,1] and backward [2,3]
 	int evok;                 // events created
 	int evrec;                // bit 0: forward pair recorded, bit 1: backward pair
@@ -278,7 +277,7 @@ static __device__ void box_flush(const Geo &g, const Box &b, const double *sacc,
 
 // rho += Dep(r) for the particles of the block
 __global__ __launch_bounds__(CPIC_BLOCK)
-void k_adj_deposit(Geo g, AdjSpecies k, int64_t n, const int32_t *__restrict__ sp,
+void k_adj_deposit(Geo g, AdjSpecies k, int64_t n, const uint8_t *__restrict__ sp,
 		const double *__restrict__ x, const double *__restrict__ y, double *__restrict__ rho)
 {
 	__shared__ double sacc[ADJ_BOX_NODES];
@@ -315,7 +314,7 @@ void k_adj_deposit(Geo g, AdjSpecies k, int64_t n, const int32_t *__restrict__ s
 template <bool DEP, int PPT>
 __global__ __launch_bounds__(CPIC_BLOCK)
 void k_adj_push(Geo g, AdjSpecies k, int set_r, double dtp, int64_t n,
-		const int32_t *__restrict__ sp, const double *x, const double *y, double *xo,
+		const uint8_t *__restrict__ sp, const double *x, const double *y, double *xo,
 		double *yo, double *__restrict__ ux, double *__restrict__ uy,
 		const double2 *__restrict__ E, double *__restrict__ rho_next, int *derr)
 {
@@ -434,7 +433,7 @@ static_assert(ADJ_CHUNK % REV_CHUNK == 0, "reverse blocks split the sort's chunk
 template <bool PEND>
 __global__ __launch_bounds__(CPIC_BLOCK)
 void k_adj_rev_a(Geo g, AdjSpecies k, int set_r, double dtp, int64_t n,
-		const int32_t *__restrict__ sp, const double *__restrict__ x,
+		const uint8_t *__restrict__ sp, const double *__restrict__ x,
 		const double *__restrict__ y, const double2 *__restrict__ E, double *__restrict__ lx,
 		double *__restrict__ ly, double *__restrict__ lux, double *__restrict__ luy,
 		double2 *__restrict__ lE, const double *__restrict__ bx, const double *__restrict__ by,
@@ -544,7 +543,7 @@ void k_adj_field(Geo g, const double2 *__restrict__ lE, const double *__restrict
 // lr += c * grad Gat(lrho)(r) for the last iteration of the sweep (the
 // others are applied by the next k_adj_rev_a)
 __global__ __launch_bounds__(CPIC_BLOCK)
-void k_adj_rev_b(Geo g, AdjSpecies k, int64_t n, const int32_t *__restrict__ sp,
+void k_adj_rev_b(Geo g, AdjSpecies k, int64_t n, const uint8_t *__restrict__ sp,
 		const double *__restrict__ x, const double *__restrict__ y,
 		const double *__restrict__ lrho, double *__restrict__ lx, double *__restrict__ ly)
 {
@@ -555,6 +554,229 @@ void k_adj_rev_b(Geo g, AdjSpecies k, int64_t n, const int32_t *__restrict__ sp,
 		rev_b_term(g, k.c[sp[i]], x[i], y[i], lrho, ax, ay);
 		lx[i] = ax;
 		ly[i] = ay;
+	}
+}
+
+// ------------------------------------------------------ particle order ---
+//
+// The particles are kept in the order of their initial cell, and within each
+// run of ADJ_CHUNK positions the cells are taken round-robin: one particle of
+// every cell that still has one, per round, so that the 64 consecutive
+// particles of a wavefront lie in different cells and their deposit atomics
+// spread over the LDS banks (sort_by_cell_rr() in host_sort.h is the
+// sequential statement of it).  Counted, scanned and placed on the device;
+// 4,194,304 particles at 256^2, a forward and a backward from host arrays:
+// 69.4 ms with the order made, applied and undone by 16 host threads, 48.2 ms so.
+
+#define ADJ_SCAN 2048             // cells per block of the scan
+#define ADJ_DERR_INPUT 0x100      // derr: a particle outside the box or not finite
+
+// cell[i] of the caller's particle i, rank[i] its number among the particles
+// of its cell, cnt[cell] their count
+__global__ __launch_bounds__(CPIC_BLOCK)
+void k_adj_cells(Geo g, int64_t n, const double *__restrict__ raw, int32_t *__restrict__ cell,
+		int32_t *__restrict__ rank, int32_t *__restrict__ cnt, int *__restrict__ derr)
+{
+	bool bad = false;
+	for(int64_t i = blockIdx.x * (int64_t) blockDim.x + threadIdx.x; i < n;
+			i += (int64_t) gridDim.x * blockDim.x)
+	{
+		const double x = raw[i], y = raw[n + i];
+		int c = 0;
+		if(x >= 0.0 && x <= g.L0 && y >= 0.0 && y <= g.L1)
+			c = min((int) (y * g.idy), g.ny - 1) * g.nx + min((int) (x * g.idx), g.nx - 1);
+		else
+			bad = true;
+		if(!isfinite(raw[2 * n + i]) || !isfinite(raw[3 * n + i]))
+			bad = true;
+		cell[i] = c;
+		rank[i] = atomicAdd(&cnt[c], 1);
+	}
+	if(bad)
+		atomicOr(derr, ADJ_DERR_INPUT);
+}
+
+// Sum of v over the threads before this one, and over all of them (into *all).
+static __device__ __forceinline__ int64_t block_before(int64_t v, int64_t *s_w, int64_t *all)
+{
+	const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
+	int64_t x = v;
+	for(int off = 1; off < 64; off <<= 1)
+	{
+		int64_t o = __shfl_up((long long) x, off);
+		if(lane >= off)
+			x += o;
+	}
+	__syncthreads();
+	if(lane == 63)
+		s_w[wid] = x;
+	__syncthreads();
+	int64_t before = x - v, t = 0;
+	for(int w = 0; w < nw; w++)
+	{
+		if(w < wid)
+			before += s_w[w];
+		t += s_w[w];
+	}
+	*all = t;
+	return before;
+}
+
+// Particles in each ADJ_SCAN cells
+__global__ __launch_bounds__(CPIC_BLOCK)
+void k_adj_scan_sums(int64_t cells, const int32_t *__restrict__ cnt, int64_t *__restrict__ part)
+{
+	__shared__ int64_t s_w[CPIC_BLOCK / 64];
+	int64_t sum = 0, all;
+	for(int64_t k = threadIdx.x; k < ADJ_SCAN; k += CPIC_BLOCK)
+	{
+		int64_t c = (int64_t) blockIdx.x * ADJ_SCAN + k;
+		sum += c < cells ? cnt[c] : 0;
+	}
+	block_before(sum, s_w, &all);
+	if(threadIdx.x == 0)
+		part[blockIdx.x] = all;
+}
+
+// Exclusive scan of the n sums, one block
+__global__ __launch_bounds__(1024)
+void k_adj_scan_part(int n, int64_t *__restrict__ part)
+{
+	__shared__ int64_t s_w[1024 / 64];
+	int64_t carry = 0;
+	for(int k = 0; k < n; k += 1024)
+	{
+		const int i = k + (int) threadIdx.x;
+		int64_t v = i < n ? part[i] : 0, all;
+		int64_t b = block_before(v, s_w, &all);
+		if(i < n)
+			part[i] = carry + b;
+		carry += all;
+	}
+}
+
+// start[c]: particles in the cells before c
+__global__ __launch_bounds__(CPIC_BLOCK)
+void k_adj_scan_starts(int64_t cells, const int32_t *__restrict__ cnt,
+		const int64_t *__restrict__ part, int64_t *__restrict__ start)
+{
+	__shared__ int64_t s_w[CPIC_BLOCK / 64];
+	constexpr int PER = ADJ_SCAN / CPIC_BLOCK;
+	const int64_t c0 = (int64_t) blockIdx.x * ADJ_SCAN + (int64_t) threadIdx.x * PER;
+	int v[PER];
+	int64_t sum = 0, all;
+	for(int k = 0; k < PER; k++)
+	{
+		v[k] = c0 + k < cells ? cnt[c0 + k] : 0;
+		sum += v[k];
+	}
+	int64_t at = part[blockIdx.x] + block_before(sum, s_w, &all);
+	for(int k = 0; k < PER; k++)
+	{
+		if(c0 + k < cells)
+			start[c0 + k] = at;
+		at += v[k];
+	}
+}
+
+// The particles by cell: position j holds the caller's particle order[j], of
+// cell scell[j]
+__global__ __launch_bounds__(CPIC_BLOCK)
+void k_adj_place(int64_t n, const int32_t *__restrict__ cell, const int32_t *__restrict__ rank,
+		const int64_t *__restrict__ start, int64_t *__restrict__ order,
+		int32_t *__restrict__ scell)
+{
+	for(int64_t i = blockIdx.x * (int64_t) blockDim.x + threadIdx.x; i < n;
+			i += (int64_t) gridDim.x * blockDim.x)
+	{
+		const int c = cell[i];
+		const int64_t j = start[c] + rank[i];
+		order[j] = i;
+		scell[j] = c;
+	}
+}
+
+// Takes the cells of one chunk round-robin and fetches the state in the
+// resulting order.  The r-th particle (from 0) of the chunk's q-th cell follows the
+// first r particles of every cell, and the r-th ones of the cells before it.
+__global__ __launch_bounds__(CPIC_BLOCK)
+void k_adj_robin(int64_t n, const int64_t *__restrict__ order, const int32_t *__restrict__ scell,
+		const double *__restrict__ raw, const uint8_t *__restrict__ sp0,
+		int64_t *__restrict__ perm, double *__restrict__ x, double *__restrict__ y,
+		double *__restrict__ ux, double *__restrict__ uy, uint8_t *__restrict__ sp)
+{
+	__shared__ int s_cell[ADJ_CHUNK], s_head[ADJ_CHUNK + 1];
+	__shared__ int64_t s_w[CPIC_BLOCK / 64];
+	const int64_t c0 = (int64_t) blockIdx.x * ADJ_CHUNK;
+	const int m = (int) min((int64_t) ADJ_CHUNK, n - c0);
+	for(int j = threadIdx.x; j < m; j += CPIC_BLOCK)
+		s_cell[j] = scell[c0 + j];
+	__syncthreads();
+	// the chunk's cells: s_head[q] is the q-th one's first position
+	const int j0 = threadIdx.x * ADJ_PPT;
+	int q[ADJ_PPT], heads = 0;
+	for(int u = 0; u < ADJ_PPT; u++)
+	{
+		const int j = j0 + u;
+		if(j < m && (j == 0 || s_cell[j] != s_cell[j - 1]))
+			heads++;
+		q[u] = heads;
+	}
+	int64_t all;
+	const int before = (int) block_before(heads, s_w, &all);
+	const int nq = (int) all;
+	for(int u = 0; u < ADJ_PPT; u++)
+	{
+		const int j = j0 + u;
+		q[u] += before - 1;
+		if(j < m && (j == 0 || s_cell[j] != s_cell[j - 1]))
+			s_head[q[u]] = j;
+	}
+	if(threadIdx.x == 0)
+		s_head[nq] = m;
+	__syncthreads();
+	int r[ADJ_PPT], f[ADJ_PPT];
+	for(int u = 0; u < ADJ_PPT; u++)
+	{
+		r[u] = j0 + u < m ? j0 + u - s_head[q[u]] : 0;
+		f[u] = 0;
+	}
+	for(int k = 0, h = 0; k < nq; k++)
+	{
+		const int hn = s_head[k + 1], len = hn - h;
+		h = hn;
+#pragma unroll
+		for(int u = 0; u < ADJ_PPT; u++)
+			f[u] += min(len, r[u]) + (k < q[u] && len > r[u] ? 1 : 0);
+	}
+	for(int u = 0; u < ADJ_PPT; u++)
+	{
+		if(j0 + u >= m)
+			continue;
+		const int64_t i = order[c0 + j0 + u], o = c0 + f[u];
+		perm[o] = i;
+		x[o] = raw[i];
+		y[o] = raw[n + i];
+		ux[o] = raw[2 * n + i];
+		uy[o] = raw[3 * n + i];
+		sp[o] = sp0[i];
+	}
+}
+
+// Four arrays in sorted order -> the caller's order (out: 4 arrays of n)
+__global__ __launch_bounds__(CPIC_BLOCK)
+void k_adj_unsort(int64_t n, const int64_t *__restrict__ perm, const double *__restrict__ a0,
+		const double *__restrict__ a1, const double *__restrict__ a2,
+		const double *__restrict__ a3, double *__restrict__ out)
+{
+	for(int64_t j = blockIdx.x * (int64_t) blockDim.x + threadIdx.x; j < n;
+			j += (int64_t) gridDim.x * blockDim.x)
+	{
+		const int64_t i = perm[j];
+		out[i] = a0[j];
+		out[n + i] = a1[j];
+		out[2 * n + i] = a2[j];
+		out[3 * n + i] = a3[j];
 	}
 }
 
@@ -583,7 +805,7 @@ adj_free(cpic_adj *a)
 		return;
 	if(a->d)
 		hipStreamSynchronize(a->d->stream);
-	hipFree(a->sp); hipFree(a->x); hipFree(a->y); hipFree(a->ux); hipFree(a->uy);
+	hipFree(a->sp); hipFree(a->sp0); hipFree(a->perm); hipFree(a->x); hipFree(a->y); hipFree(a->ux); hipFree(a->uy);
 	hipFree(a->rho[0]); hipFree(a->rho[1]); hipFree(a->phi); hipFree(a->psi); hipFree(a->lrho);
 	hipFree(a->E); hipFree(a->lE);
 	hipFree(a->lx); hipFree(a->ly); hipFree(a->lux); hipFree(a->luy);
@@ -594,10 +816,6 @@ adj_free(cpic_adj *a)
 	if(a->evok)
 		for(int i = 0; i < 4; i++)
 			hipEventDestroy(a->ev[i]);
-	free(a->hsp);
-	free(a->perm);
-	if(a->hbuf)
-		hipHostFree(a->hbuf);
 	if(a->d)
 		cpic_dev_destroy(a->d);
 	free(a);
@@ -649,7 +867,19 @@ cpic_adj_create(const cpic_dev_desc_t *desc, int64_t n, const int32_t *species,
 	species_consts(desc, desc->dt, &a->k[1]);
 	int64_t nodes = (int64_t) a->g.nx * a->g.ny;
 	size_t pn = sizeof(double) * (size_t) n, gn = sizeof(double) * (size_t) nodes;
-	if(hipMalloc(&a->sp, sizeof(int32_t) * n) != hipSuccess ||
+	uint8_t *sp8 = (uint8_t *) malloc((size_t) n);
+	if(!sp8)
+	{
+		adj_free(a);
+		return CPIC_ENOMEM;
+	}
+	for(int64_t i = 0; i < n; i++)
+		sp8[i] = (uint8_t) species[i];
+	if(hipMalloc(&a->sp, (size_t) n) != hipSuccess ||
+			hipMalloc(&a->sp0, (size_t) n) != hipSuccess ||
+			hipMemcpy(a->sp0, sp8, (size_t) n, hipMemcpyHostToDevice) != hipSuccess ||
+			hipMalloc(&a->perm, sizeof(int64_t) * (size_t) n) != hipSuccess ||
+			hipMalloc(&a->wk, 4 * pn) != hipSuccess ||
 			hipMalloc(&a->x, pn) != hipSuccess || hipMalloc(&a->y, pn) != hipSuccess ||
 			hipMalloc(&a->ux, pn) != hipSuccess || hipMalloc(&a->uy, pn) != hipSuccess ||
 			hipMalloc(&a->lx, pn) != hipSuccess || hipMalloc(&a->ly, pn) != hipSuccess ||
@@ -660,20 +890,11 @@ cpic_adj_create(const cpic_dev_desc_t *desc, int64_t n, const int32_t *species,
 			hipMalloc(&a->E, 2 * gn) != hipSuccess || hipMalloc(&a->lE, 4 * gn) != hipSuccess ||
 			hipMalloc(&a->derr, sizeof(int)) != hipSuccess)
 	{
+		free(sp8);
 		adj_free(a);
 		return CPIC_ENOMEM;
 	}
-	a->hsp = (int32_t *) malloc(sizeof(int32_t) * (size_t) n);
-	a->perm = (int64_t *) malloc(sizeof(int64_t) * (size_t) n);
-	if(hipHostMalloc((void **) &a->hbuf, sizeof(double) * 4 * (size_t) n, hipHostMallocDefault)
-			!= hipSuccess)
-		a->hbuf = NULL;
-	if(!a->hsp || !a->perm || !a->hbuf)
-	{
-		adj_free(a);
-		return CPIC_ENOMEM;
-	}
-	memcpy(a->hsp, species, sizeof(int32_t) * n);
+	free(sp8);
 	for(int i = 0; i < 4; i++)
 		if(hipEventCreate(&a->ev[i]) != hipSuccess)
 		{
@@ -821,18 +1042,40 @@ copy_state(cpic_adj *a, double *dst, const double *x, const double *y, const dou
 	return 0;
 }
 
-// perm: the particles in the order of their cell (iy*nx + ix), counting
-// sort, stable; the deposits' LDS boxes rely on neighbours in this order
-// being neighbours on the grid.
+// The caller's particles, in wk, into the state in sorted order (see "particle
+// order"); CPIC_EINVAL, with the state as it was, if one is outside the box or
+// not finite.  The reverse sweep's buffers hold the intermediate arrays.
 static int
-sort_by_cell(cpic_adj *a, const double *x, const double *y)
+sort_in(cpic_adj *a)
 {
-	// Within each block's chunk (same cells, so the same LDS box) the cells
-	// are taken round-robin: the 64 consecutive particles of a wavefront
-	// then lie in different cells, and their deposit atomics spread over the
-	// LDS banks instead of piling onto the 4 nodes of one cell.
-	return sort_by_cell_rr(a->n, x, y, a->g.idx, a->g.idy, a->g.nx, a->g.ny, ADJ_CHUNK,
-			a->perm) ? CPIC_ENOMEM : 0;
+	const int64_t n = a->n, cells = (int64_t) a->g.nx * a->g.ny;
+	int32_t *cell = (int32_t *) a->ly, *rank = cell + n, *scell = (int32_t *) a->lux;
+	int32_t *cnt = (int32_t *) a->lrho;
+	int64_t *order = (int64_t *) a->lx, *start = (int64_t *) a->psi, *part = (int64_t *) a->rho[1];
+	const int sb = (int) ((cells + ADJ_SCAN - 1) / ADJ_SCAN);
+	const dim3 block(CPIC_BLOCK), pb(pblocks(n));
+	hipStream_t st = a->d->stream;
+	int ret, e = 0;
+	// cells is even: both grid sides are powers of two from 2 up
+	if((ret = zero(a, (double *) cnt, cells / 2)))
+		return ret;
+	HIPCHK(hipMemsetAsync(a->derr, 0, sizeof(int), st));
+	hipLaunchKernelGGL(k_adj_cells, pb, block, 0, st, a->g, n, (const double *) a->wk, cell, rank,
+			cnt, a->derr);
+	hipLaunchKernelGGL(k_adj_scan_sums, dim3(sb), block, 0, st, cells, cnt, part);
+	hipLaunchKernelGGL(k_adj_scan_part, dim3(1), dim3(1024), 0, st, sb, part);
+	hipLaunchKernelGGL(k_adj_scan_starts, dim3(sb), block, 0, st, cells, cnt, part, start);
+	hipLaunchKernelGGL(k_adj_place, pb, block, 0, st, n, cell, rank, start, order, scell);
+	HIPCHK(hipGetLastError());
+	HIPCHK(hipMemcpyAsync(&e, a->derr, sizeof(int), hipMemcpyDeviceToHost, st));
+	HIPCHK(hipStreamSynchronize(st));
+	if(e & ADJ_DERR_INPUT)
+		return CPIC_EINVAL;
+	hipLaunchKernelGGL(k_adj_robin, dim3(chunks(n)), block, 0, st, n, order, scell,
+			(const double *) a->wk, (const uint8_t *) a->sp0, a->perm, a->x, a->y, a->ux, a->uy,
+			a->sp);
+	HIPCHK(hipGetLastError());
+	return 0;
 }
 
 // Device arrays in sorted order -> host arrays in the caller's order.
@@ -840,15 +1083,16 @@ static int
 download_unsorted(cpic_adj *a, double *const *src, double *const *dst)
 {
 	const int64_t n = a->n;
-	size_t pn = sizeof(double) * (size_t) n;
+	DlRange r[4];
+	int nr = 0;
+	hipLaunchKernelGGL(k_adj_unsort, dim3(pblocks(n)), dim3(CPIC_BLOCK), 0, a->d->stream, n,
+			(const int64_t *) a->perm, (const double *) src[0], (const double *) src[1],
+			(const double *) src[2], (const double *) src[3], a->wk);
+	HIPCHK(hipGetLastError());
 	for(int c = 0; c < 4; c++)
 		if(dst[c])
-			HIPCHK(hipMemcpyAsync(a->hbuf + c * n, src[c], pn, hipMemcpyDeviceToHost, a->d->stream));
-	HIPCHK(hipStreamSynchronize(a->d->stream));
-	for(int c = 0; c < 4; c++)
-		if(dst[c])
-			scatter_perm(n, a->perm, (const double *) (a->hbuf + c * n), dst[c]);
-	return 0;
+			r[nr++] = {dst[c], a->wk + c * n, sizeof(double) * (size_t) n};
+	return nr ? cpic_download(a->d, nr, r) : 0;
 }
 
 // Whether this forward keeps its position history, whose memory is then there.
@@ -881,42 +1125,15 @@ cpic_adj_forward(cpic_adj_t *a, const double *x, const double *y, const double *
 	int ret, cur = 0;
 	if(!a || !x || !y || !ux || !uy || nsteps < 1 || checkpoint_every < 1)
 		return CPIC_EINVAL;
-	std::atomic<int> invalid(0);
-	parallel_ranges(a->n, host_threads(a->n, 1 << 16), [&](int, int64_t lo, int64_t hi) {
-		for(int64_t i = lo; i < hi; i++)
-			if(!(x[i] >= 0.0 && x[i] <= a->g.L0 && y[i] >= 0.0 && y[i] <= a->g.L1) ||
-					!std::isfinite(ux[i]) || !std::isfinite(uy[i]))
-			{
-				invalid = 1;
-				return;
-			}
-	});
-	if(invalid)
-		return CPIC_EINVAL;
 	hipSetDevice(a->d->device);
 	int64_t K = checkpoint_every, nck = (nsteps + K - 1) / K, n = a->n;
 	if((ret = grow(&a->hist, &a->histcap, nsteps)))
 		return ret;
-	if((ret = sort_by_cell(a, x, y)))
+	const size_t pn = sizeof(double) * (size_t) n;
+	const DlRange up[4] = {{a->wk, x, pn}, {a->wk + n, y, pn}, {a->wk + 2 * n, ux, pn},
+		{a->wk + 3 * n, uy, pn}};
+	if((ret = cpic_upload(a->d, 4, up)) || (ret = sort_in(a)))
 		return ret;
-	size_t pn = sizeof(double) * (size_t) n;
-	const double *src[4] = {x, y, ux, uy};
-	double *dev[4] = {a->x, a->y, a->ux, a->uy};
-	int32_t *ssp = (int32_t *) malloc(sizeof(int32_t) * (size_t) n);
-	if(!ssp)
-		return CPIC_ENOMEM;
-	gather_perm(n, a->perm, (const int32_t *) a->hsp, ssp);
-	hipError_t e = hipMemcpy(a->sp, ssp, sizeof(int32_t) * n, hipMemcpyHostToDevice);
-	free(ssp);
-	if(e != hipSuccess)
-		return CPIC_EHIP;
-	for(int c = 0; c < 4; c++)
-	{
-		double *h = a->hbuf + c * n;
-		gather_perm(n, a->perm, src[c], h);
-		HIPCHK(hipMemcpyAsync(dev[c], h, pn, hipMemcpyHostToDevice, a->d->stream));
-	}
-	HIPCHK(hipMemsetAsync(a->derr, 0, sizeof(int), a->d->stream));
 	a->have = 0;
 	a->evrec = 0;             // a backward belongs to the forward before it
 	// the field history, when it fits: each iteration's rho and E are
@@ -1059,11 +1276,6 @@ cpic_adj_backward(cpic_adj_t *a, double dloss, double *gx, double *gy, double *g
 	if((!ph && (ret = grow(&a->seg, &a->segcap, 2 * n * (Kseg - 1)))) ||
 			(!fh && (ret = grow(&a->segf, &a->segfcap, 3 * nodes * Kseg))))
 		return ret;
-	if(!a->wk && hipMalloc(&a->wk, sizeof(double) * 4 * (size_t) n) != hipSuccess)
-	{
-		a->wk = NULL;
-		return CPIC_ENOMEM;
-	}
 	a->evrec &= ~2;
 	HIPCHK(hipEventRecord(a->ev[2], a->d->stream));
 	// both lE buffers start at zero; each iteration's k_adj_field zeroes the

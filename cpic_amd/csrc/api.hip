@@ -522,17 +522,17 @@ cpic_dev_destroy(cpic_dev_t *d)
 // ---------------------------------------------------------- downloads ---
 
 // Copies device ranges to ordinary host memory after the work queued on the
-// handle's stream.  Copying straight into pageable memory runs at ~9 GB/s:
+// handle's stream, or (up) the other way.  Copying straight into pageable memory runs at ~9 GB/s:
 // the runtime's own staging is one thread's, and for a fresh destination
 // that thread also takes every page fault.  Here the ranges go, DL_CHUNK
 // bytes at a time, through two pinned buffers; while one is filled by DMA,
 // the threads copy the other out, each taking its share of the chunk's pages
 // (and faults).  Small downloads copy on the calling thread: starting threads
 // would cost more than they save.
-int
-cpic_download(cpic_dev *d, int nr, const DlRange *r)
+static int
+copy_ranges(cpic_dev *d, int nr, const DlRange *r, bool up)
 {
-	struct Piece { size_t at, dst_off, bytes; int range; };
+	struct Piece { size_t at, off, bytes; int range; };
 	std::vector<Piece> pieces;
 	std::vector<size_t> first;         // pieces of chunk c: [first[c], first[c+1])
 	size_t total = 0, fill = DL_CHUNK;
@@ -568,32 +568,48 @@ cpic_download(cpic_dev *d, int nr, const DlRange *r)
 	const int nt = host_threads((int64_t) total, (int64_t) 1 << 20);
 	std::atomic<int> ready(0), fail(0);
 	std::atomic<int> done[2] = {{0}, {0}};      // shares copied out of each buffer
+	int workers = 0;
 	// thread t of n copies its share of every piece of chunk c
-	auto copy_out = [&](int c, int t, int n) {
-		const char *b = d->pin + (size_t) (c & 1) * DL_CHUNK;
+	auto copy = [&](int c, int t, int n) {
+		char *b = d->pin + (size_t) (c & 1) * DL_CHUNK;
 		for(size_t k = first[c]; k < first[c + 1]; k++)
 		{
 			const Piece &p = pieces[k];
 			size_t lo = (p.bytes * (size_t) t / (size_t) n) & ~(size_t) 63;
 			size_t hi = t + 1 == n ? p.bytes :
 				(p.bytes * (size_t) (t + 1) / (size_t) n) & ~(size_t) 63;
-			memcpy((char *) r[p.range].dst + p.dst_off + lo, b + p.at + lo, hi - lo);
+			if(up)
+				memcpy(b + p.at + lo, (const char *) r[p.range].src + p.off + lo, hi - lo);
+			else
+				memcpy((char *) r[p.range].dst + p.off + lo, b + p.at + lo, hi - lo);
 		}
 	};
-	auto fetch = [&](int c) -> hipError_t {
+	// queues the DMA of chunk c
+	auto dma = [&](int c) -> hipError_t {
 		char *b = d->pin + (size_t) (c & 1) * DL_CHUNK;
-		for(size_t k = first[c]; k < first[c + 1]; k++)
+		hipError_t e = hipSuccess;
+		for(size_t k = first[c]; k < first[c + 1] && e == hipSuccess; k++)
 		{
 			const Piece &p = pieces[k];
-			hipError_t e = hipMemcpyAsync(b + p.at, (const char *) r[p.range].src + p.dst_off,
-					p.bytes, hipMemcpyDeviceToHost, d->stream);
-			if(e != hipSuccess)
-				return e;
+			if(up)
+				e = hipMemcpyAsync((char *) r[p.range].dst + p.off, b + p.at, p.bytes,
+						hipMemcpyHostToDevice, d->stream);
+			else
+				e = hipMemcpyAsync(b + p.at, (const char *) r[p.range].src + p.off, p.bytes,
+						hipMemcpyDeviceToHost, d->stream);
 		}
-		return hipStreamSynchronize(d->stream);
+		return e;
+	};
+	// shares of chunk c without a thread of their own, then those of the threads
+	auto finish = [&](int c) {
+		for(int t = workers; t < nt; t++)
+			copy(c, t, nt);
+	};
+	auto wait_done = [&](int c) {
+		while(done[c & 1].load(std::memory_order_acquire) < workers * (c / 2 + 1))
+			std::this_thread::yield();
 	};
 	std::vector<std::thread> th;
-	int workers = 0;
 	try
 	{
 		th.reserve((size_t) nt);
@@ -608,7 +624,7 @@ cpic_download(cpic_dev *d, int nr, const DlRange *r)
 							return;
 						std::this_thread::yield();
 					}
-					copy_out(c, t, nt);
+					copy(c, t, nt);
 					done[c & 1].fetch_add(1, std::memory_order_release);
 				}
 			});
@@ -620,25 +636,52 @@ cpic_download(cpic_dev *d, int nr, const DlRange *r)
 		// the calling thread copies the other shares
 	}
 	hipError_t e = hipSuccess;
-	for(int c = 0; c < nchunks && e == hipSuccess; c++)
+	if(up)
 	{
-		// every share of the buffer's earlier chunks has been copied out
-		while(done[c & 1].load(std::memory_order_acquire) < workers * (c / 2))
-			std::this_thread::yield();
-		if((e = fetch(c)) != hipSuccess)
-			break;
-		ready.store(c + 1, std::memory_order_release);
-		// shares without a thread of their own
-		for(int t = workers; t < nt; t++)
-			copy_out(c, t, nt);
+		// a chunk's DMA runs while the next one's shares are copied in
+		ready.store(2, std::memory_order_release);
+		for(int c = 0; c < nchunks && e == hipSuccess; c++)
+		{
+			finish(c);
+			wait_done(c);
+			if(c > 0 && (e = hipStreamSynchronize(d->stream)) != hipSuccess)
+				break;
+			if(c > 0)
+				ready.store(c + 2, std::memory_order_release);
+			e = dma(c);
+		}
+		if(e == hipSuccess)
+			e = hipStreamSynchronize(d->stream);
 	}
+	else
+		for(int c = 0; c < nchunks && e == hipSuccess; c++)
+		{
+			if(c > 1)
+				wait_done(c - 2);
+			if((e = dma(c)) != hipSuccess || (e = hipStreamSynchronize(d->stream)) != hipSuccess)
+				break;
+			ready.store(c + 1, std::memory_order_release);
+			finish(c);
+		}
 	if(e != hipSuccess)
 		fail = 1;
 	for(auto &x : th)
 		x.join();
 	if(e != hipSuccess)
-		fprintf(stderr, "cpic_hip: download failed: %s\n", hipGetErrorString(e));
+		fprintf(stderr, "cpic_hip: host copy failed: %s\n", hipGetErrorString(e));
 	return e == hipSuccess ? 0 : CPIC_EHIP;
+}
+
+int
+cpic_download(cpic_dev *d, int nr, const DlRange *r)
+{
+	return copy_ranges(d, nr, r, false);
+}
+
+int
+cpic_upload(cpic_dev *d, int nr, const DlRange *r)
+{
+	return copy_ranges(d, nr, r, true);
 }
 
 // ---------------------------------------------------------- particles ---

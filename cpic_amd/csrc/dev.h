@@ -144,7 +144,8 @@ struct StepState {
 	long long pad[7];
 };
 
-// One contiguous device range of a download and its host destination.
+// One contiguous range of a download (src on the device) or an upload (dst on
+// the device).
 struct DlRange {
 	void *dst;
 	const void *src;
@@ -241,7 +242,7 @@ struct cpic_dev {
 	int graph_ok;
 	int capturing;           // inside hipStreamBeginCapture/EndCapture
 
-	// downloads: pinned bounce buffers (2 x DL_CHUNK bytes) and the particle
+	// host copies: pinned bounce buffers (2 x DL_CHUNK bytes) and the particle
 	// downloads' device workspace, both kept between calls
 	char *pin;
 	char *dl;
@@ -283,6 +284,7 @@ int cpic_parts_deposit(cpic_dev *d, double *rho_out);
 int cpic_parts_gather(cpic_dev *d);
 int cpic_parts_download(cpic_dev *d, int plasma, int species, int sorted, cpic_particles_t *out);
 int cpic_download(cpic_dev *d, int n, const DlRange *r);
+int cpic_upload(cpic_dev *d, int n, const DlRange *r);
 int cpic_parts_cell_counts(cpic_dev *d, int plasma, int species, int64_t *counts);
 int cpic_parts_alloc(cpic_dev *d, int which, int64_t cap);
 void cpic_parts_free(cpic_dev *d, int which);
