@@ -1144,6 +1144,8 @@ graph_steps(cpic_dev *d, int64_t iter)
 		d->last_iter = iter + 1;
 	}
 	HIPCHK(hipGraphLaunch(d->graph, d->stream));
+	// the replayed solves renew phi, whatever has read E since the capture
+	d->E_stale = 1;
 	return 0;
 }
 
