@@ -958,10 +958,7 @@ deposit(cpic_adj *a, const double *x, const double *y, double *rho)
 static int
 fields(cpic_adj *a, const double *rho, double *w, double *rho_zero, double2 *E)
 {
-	int ret;
-	if((ret = cpic_solve_ptr_energy(a->d, rho, a->phi, rho_zero, w)))
-		return ret;
-	return cpic_efield_ptr(a->d, a->phi, E);
+	return cpic_solve_ptr_E(a->d, rho, a->phi, rho_zero, w, E);
 }
 
 // one forward iteration from positions (x, y), velocities (ux, uy) and
@@ -1370,6 +1367,15 @@ cpic_adj_backward(cpic_adj_t *a, double dloss, double *gx, double *gy, double *g
 						a->g, a->k[first ? 0 : 1], first ? 0 : 1, dtp, n, a->sp, sx, sy,
 						(const double2 *) seg_E(it, it0), a->lx, a->ly, a->lux, a->luy, lE,
 						(const double *) NULL, (const double *) NULL, (const double *) NULL);
+			if(a->d->fft_small)
+			{
+				if(hipGetLastError() != hipSuccess)
+					ret = CPIC_EHIP;
+				else
+					ret = cpic_solve_transposed_small(a->d, lE, seg_rho(it, it0),
+							dloss * a->g.e0, lE_next, a->lrho);
+				continue;
+			}
 			hipLaunchKernelGGL(k_adj_field, dim3(pblocks(nodes)), dim3(CPIC_BLOCK), 0,
 					a->d->stream, a->g, (const double2 *) lE, seg_rho(it, it0),
 					dloss * a->g.e0, a->psi, lE_next);

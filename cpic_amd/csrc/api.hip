@@ -430,6 +430,7 @@ batch_create(const cpic_dev_desc_t *descs, int P, cpic_dev_t **out)
 	d->nodeblocks = (int) nblk;
 	d->lds_rows = lds_rows;
 	d->lds_cols = lds_cols;
+	d->fft_small = cpic_solve_is_small(d);
 	d->lds_push = cpic_push_lds(d);
 	for(p = 0; p < P; p++)
 		if(d->hgeo[p].ns > d->maxns)

@@ -180,6 +180,7 @@ struct cpic_dev {
 	int rowblocks, colblocks, nodeblocks;
 	int fft_nt_row, fft_nt_col;   // threads per block of the FFT row and column passes
 	size_t lds_push, lds_rows, lds_cols;
+	int fft_small;           // every plasma's solve is one workgroup's
 	int phi_apart;           // the push's potential region has LDS of its own
 
 	// fields
@@ -274,6 +275,11 @@ int cpic_solve_ptr_zero(cpic_dev *d, const double *rho, double *phi, double *rho
 // energy[p] (summed over the spectrum by the column pass)
 int cpic_solve_ptr_energy(cpic_dev *d, const double *rho, double *phi, double *rho_zero,
 		double *energy);
+int cpic_solve_ptr_E(cpic_dev *d, const double *rho, double *phi, double *rho_zero,
+		double *energy, void *E);
+int cpic_solve_is_small(const cpic_dev *d);
+int cpic_solve_transposed_small(cpic_dev *d, const double2 *lE, const double *rho, double srho,
+		double2 *lE_zero, double *lrho);
 int cpic_efield_ptr(cpic_dev *d, const double *phi, void *E);
 int cpic_efield(cpic_dev *d);
 int cpic_parts_init(cpic_dev *d);

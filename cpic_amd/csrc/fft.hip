@@ -92,6 +92,34 @@ static __device__ __forceinline__ TwRef tw_fill(TwLds &t, const double2 *__restr
 	return r;
 }
 
+static __host__ __device__ void twiddle(int64_t k, int64_t n, double *c, double *s);
+
+// The same tables computed instead of copied, entry k by thread t = k mod the
+// block size.
+static __device__ __forceinline__ TwRef tw_make(TwLds &tl, int lgN, int t)
+{
+	const int a = (lgN + 1) >> 1, half = 1 << (lgN - 1);
+	for(int k = t; k < (1 << a) + (1 << (lgN - a)); k += blockDim.x)
+	{
+		const bool lo = k < (1 << a);
+		const int idx = lo ? k : (k - (1 << a)) << a;
+		const bool neg = !lo && idx >= half;
+		double2 w;
+		twiddle(neg ? idx - half : idx, 1 << lgN, &w.x, &w.y);
+		if(neg)
+		{
+			w.x = -w.x;
+			w.y = -w.y;
+		}
+		(lo ? tl.lo[k] : tl.hi[k - (1 << a)]) = w;
+	}
+	TwRef r;
+	r.lo = (const LDS_AS double *) tl.lo;
+	r.hi = (const LDS_AS double *) tl.hi;
+	r.a = a;
+	return r;
+}
+
 // w = exp(sign * 2 pi i idx / N), 0 <= idx < N
 static __device__ __forceinline__ double2 twiddle_at(const TwRef &t, int idx, double sign)
 {
@@ -633,6 +661,313 @@ void k_rows_c2r(const Geo *__restrict__ geo, const int *__restrict__ pre, int P,
 	}
 }
 
+// ----------------------------------------------------- small grids ---
+//
+// A grid of up to FFT_SMALL_VALUES complex values (half its nodes) fits one
+// workgroup's LDS, so the three passes, the stencil that gives E and, for the
+// differentiable run's reverse sweep, the one before the solve are one launch of
+// one workgroup per plasma.  Bound by latency: launches, then the chain of ~11
+// stages with a barrier each.  At 64x64 one launch takes 11.3 us where the passes
+// took 5.4 + 5.7 + 4.8 (13.6 with E or the transposed stencil, which took 5.0
+// and 3.1 more); without a handle, tables included, 11.9 us instead of
+// 18.4 for four launches.  1,024 threads, not one per radix-8 butterfly: with 256
+// the elementwise steps made it 14.8 us; radix-4 stages, which keep twice
+// the threads busy, 13.1 us.  The line is at 2,048 values: 64x64 and 128x32
+// 12.0 us in one workgroup against 18.9 and 19.3, 128x64 16.3-18.5 against 17.1-18.1,
+// 128x128 29.5 against 18.3.
+#define FFT_SMALL_VALUES 2048
+#define SMALL_NT 1024
+static_assert(FFT_SMALL_VALUES <= 2 * SMALL_NT, "one radix-2 butterfly per thread");
+
+struct SmallSolve {
+	const Geo *geo;          // NULL: the grid in `one`, tables made by the kernel
+	Geo one;
+	const double *rho;
+	double *phi;
+	void *E;                 // nullable: double2 (FP64) or float2 per node
+	int e32;                 // E is float2
+	const double2 *lE;       // nullable: the right-hand side is D^T lE - srho rho
+	double srho;
+	double2 *lE_zero;        // with lE: zeroed
+	const double *costab;
+	const double2 *tw;
+	int lgN;
+	double *rho_zero;        // nullable: zeroed
+	DiagSlot *diag;          // nullable: this step's field energy
+	DiagSlot *diag_zero;     // nullable: the next step's slot, zeroed
+	int ring;
+	const StepState *st;
+	double *eout;            // nullable: field energy added to eout[p]
+};
+
+// nbat = 2^lgb transforms of length 2^lgn in place in LDS, element j of transform
+// b at b*bs + j*es.  Consecutive threads take consecutive transforms: rows
+// are an odd number of 16-byte values apart and columns one, so neither
+// direction has bank conflicts.
+template <int R>
+static __device__ __forceinline__ void small_stage(double2 *buf, int bs, int es, int lgn, int lgb,
+		int lgp, const TwRef &tw, int lgN, double sign)
+{
+	constexpr int LGR = R == 8 ? 3 : R == 4 ? 2 : 1;
+	const int nb = 1 << (lgn - LGR), p = 1 << lgp, t = threadIdx.x;
+	const int b = t & ((1 << lgb) - 1), i = t >> lgb, k = i & (p - 1);
+	const bool act = t < nb << lgb;
+	double2 v[R];
+	if(act)
+	{
+#pragma unroll
+		for(int r = 0; r < R; r++)
+			v[r] = buf[b * bs + (i + r * nb) * es];
+		if(k)
+			apply_twiddles<R>(v, twiddle_at(tw, k << (lgN - LGR - lgp), sign));
+		dft_small<R>(v, sign);
+	}
+	__syncthreads();
+	if(act)
+	{
+		const int o = b * bs + (((i - k) << LGR) + k) * es;
+#pragma unroll
+		for(int r = 0; r < R; r++)
+			buf[o + r * p * es] = v[r];
+	}
+	__syncthreads();
+}
+
+static __device__ __forceinline__ void small_fft(double2 *buf, int bs, int es, int lgn, int lgb,
+		const TwRef &tw, int lgN, double sign)
+{
+	if(lgn == 0)
+		return;
+	int lgp = first_lgr(lgn);
+	if(lgp == 1)
+		small_stage<2>(buf, bs, es, lgn, lgb, 0, tw, lgN, sign);
+	else if(lgp == 2)
+		small_stage<4>(buf, bs, es, lgn, lgb, 0, tw, lgN, sign);
+	else
+		lgp = 0;
+	for(; lgp < lgn; lgp += 3)
+		small_stage<8>(buf, bs, es, lgn, lgb, lgp, tw, lgN, sign);
+}
+
+__global__ __launch_bounds__(SMALL_NT)
+void k_solve_small(SmallSolve a)
+{
+	constexpr int NT = SMALL_NT;
+	extern __shared__ double2 sh[];
+	__shared__ TwLds s_tw;
+	__shared__ double red[NT / 64];
+	const int p = blockIdx.x, tid = threadIdx.x;
+	const bool plan = a.geo != NULL;
+	const Geo *gp = a.geo + p;
+	const int lgnx = plan ? gp->lgnx : a.one.lgnx, lgny = plan ? gp->lgny : a.one.lgny;
+	const int nx = 1 << lgnx, ny = 1 << lgny, lgm = lgnx - 1, m = nx >> 1;
+	const int stride = m + 1, n = nx * ny, lgN = a.lgN, tsh = lgN - lgnx;
+	const int64_t n0 = plan ? gp->node0 : 0;
+	const int diag0 = plan ? gp->diag0 : 0;
+	const double dx2 = plan ? 2 * gp->dx : 0.0, dy2 = plan ? 2 * gp->dy : 0.0;
+	const double invN = 1.0 / ((double) nx * (double) ny);
+	double *cosx = (double *) (sh + stride * ny), *cosy = cosx + stride;
+	const long long iter = a.st ? a.st->iter : -1;
+	double *energy = a.eout ? a.eout + p :
+		(a.diag && iter >= 0) ? &a.diag[diag0 + iter % a.ring].field : (double *) NULL;
+
+	// the right-hand side's loads go out before the tables are waited for
+	const double *__restrict__ rho = a.rho + n0;
+	double2 in[2];
+#pragma unroll
+	for(int v = 0; v < 2; v++)
+		if(tid + v * NT < m * ny)
+			in[v] = ((const double2 *) rho)[tid + v * NT];
+
+	// tables: the plan's, or made here (the entries tw_fill would copy) by the
+	// last wavefronts
+	const int back = NT - 1 - tid;
+	TwRef tw;
+	if(plan)
+	{
+		tw = tw_fill(s_tw, a.tw, lgN);
+		for(int k = tid; k < stride + ny; k += NT)
+			cosx[k] = a.costab[gp->cos0 + k];
+	}
+	else
+	{
+		tw = tw_make(s_tw, lgN, back);
+		const double cx = 2.0 * M_PI / nx, cy = 2.0 * M_PI / ny;
+		for(int k = back; k < stride + ny; k += NT)
+			cosx[k] = k < stride ? cos(cx * k) : cos(cy * (k - stride));
+	}
+	if(a.lE)
+	{
+		// D^T lE - srho rho (the transpose of the E stencil), and the other
+		// lE buffer zeroed
+		// two neighbouring nodes i, i + 1 per value
+#pragma unroll
+		for(int v = 0; v < 2; v++)
+		{
+			const int i = 2 * (tid + v * NT);
+			if(i >= n)
+				continue;
+			const int iy = i >> lgnx, ix = i & (nx - 1), row = iy << lgnx;
+			const int ym = ((iy - 1) & (ny - 1)) << lgnx, yp = ((iy + 1) & (ny - 1)) << lgnx;
+			auto psi = [&](int x, double r) {
+				const int xm = (x - 1) & (nx - 1), xp = (x + 1) & (nx - 1);
+				double lphi = (a.lE[row + xp].x - a.lE[row + xm].x) / dx2 +
+					(a.lE[yp + x].y - a.lE[ym + x].y) / dy2;
+				return lphi - a.srho * r;
+			};
+			in[v] = make_double2(psi(ix, in[v].x), psi(ix + 1, in[v].y));
+			a.lE_zero[i] = make_double2(0.0, 0.0);
+			a.lE_zero[i + 1] = make_double2(0.0, 0.0);
+		}
+	}
+#pragma unroll
+	for(int v = 0; v < 2; v++)
+	{
+		const int i = tid + v * NT;
+		if(i < m * ny)
+			sh[(i >> lgm) * stride + (i & (m - 1))] = in[v];
+	}
+	if(a.rho_zero)
+	{
+		double2 *rz = (double2 *) (a.rho_zero + n0);
+		for(int i = tid; i < m * ny; i += NT)
+			rz[i] = make_double2(0.0, 0.0);
+	}
+	__syncthreads();
+
+	small_fft(sh, stride, 1, lgm, lgny, tw, lgN, -1.0);
+	// k_rows_r2c's recombination; column 0 takes kx = 0 in its real part
+	// and kx = m in its imaginary part (see k_cols)
+	const int npair = (m >> 1) + 1;
+	for(int i = tid; i < npair << lgny; i += NT)
+	{
+		const int k = i >> lgny, b = (i & (ny - 1)) * stride;
+		if(k == 0)
+		{
+			double2 z = sh[b];
+			sh[b] = make_double2(z.x + z.y, z.x - z.y);
+		}
+		else if(2 * k == m)
+			sh[b + k].y = -sh[b + k].y;
+		else
+		{
+			double2 zk = sh[b + k], zm = sh[b + m - k];
+			double er = 0.5 * (zk.x + zm.x), ei = 0.5 * (zk.y - zm.y);
+			double dr = 0.5 * (zk.x - zm.x), di = 0.5 * (zk.y + zm.y);
+			double2 wo = cmul(make_double2(di, -dr), twiddle_at(tw, k << tsh, -1.0));
+			sh[b + k] = make_double2(er + wo.x, ei + wo.y);
+			sh[b + m - k] = make_double2(er - wo.x, -(ei - wo.y));
+		}
+	}
+	__syncthreads();
+	small_fft(sh, 1, stride, lgny, lgm, tw, lgN, -1.0);
+	// Green's function and field energy as in k_cols
+	auto green = [&](int kx, int ky) {
+		return (kx == 0 && ky == 0) ? 0.0 : 1.0 / (2.0 * (cosx[kx] + cosy[ky]) - 4.0);
+	};
+	double e = 0.0;
+	const int np0 = (ny >> 1) + 1;
+	for(int j = tid; j < np0 + (m - 1) * ny; j += NT)
+	{
+		if(j < np0)
+		{
+			const int k = j, kn = (ny - j) & (ny - 1);
+			double2 zk = sh[k * stride], zn = sh[kn * stride];
+			double2 A = make_double2(0.5 * (zk.x + zn.x), 0.5 * (zk.y - zn.y));
+			double2 B = make_double2(0.5 * (zk.y + zn.y), -0.5 * (zk.x - zn.x));
+			double a2 = A.x * A.x + A.y * A.y, b2 = B.x * B.x + B.y * B.y;
+			double ga = green(0, k), gb = green(m, k);
+			e += ga * a2 + gb * b2;
+			ga *= invN;
+			gb *= invN;
+			sh[k * stride] = make_double2(ga * A.x - gb * B.y, ga * A.y + gb * B.x);
+			if(kn != k)
+			{
+				double gan = green(0, kn), gbn = green(m, kn);
+				e += gan * a2 + gbn * b2;
+				gan *= invN;
+				gbn *= invN;
+				sh[kn * stride] = make_double2(gan * A.x + gbn * B.y, -gan * A.y + gbn * B.x);
+			}
+			continue;
+		}
+		const int i = j - np0, kx = 1 + (i >> lgny), ky = i & (ny - 1);
+		const double G = green(kx, ky);
+		double2 v = sh[ky * stride + kx];
+		e += 2.0 * G * (v.x * v.x + v.y * v.y);
+		const double gs = G * invN;
+		sh[ky * stride + kx] = make_double2(v.x * gs, v.y * gs);
+	}
+	if(energy)
+	{
+		for(int off = 32; off > 0; off >>= 1)
+			e += __shfl_down(e, off);
+		if((tid & 63) == 0)
+			red[tid >> 6] = e;
+	}
+	__syncthreads();
+	if(energy && tid == 0)
+	{
+		double t = 0.0;
+		for(int w = 0; w < NT / 64; w++)
+			t += red[w];
+		unsafeAtomicAdd(energy, t * (-0.5 * gp->e0 * invN));
+	}
+	small_fft(sh, 1, stride, lgny, lgm, tw, lgN, +1.0);
+	// k_rows_c2r's recombination
+	for(int i = tid; i < npair << lgny; i += NT)
+	{
+		const int k = i >> lgny, b = (i & (ny - 1)) * stride;
+		if(k == 0)
+		{
+			double2 z = sh[b];
+			sh[b] = make_double2(z.x + z.y, z.x - z.y);
+		}
+		else if(2 * k == m)
+			sh[b + k] = make_double2(2.0 * sh[b + k].x, -2.0 * sh[b + k].y);
+		else
+		{
+			double2 xk = sh[b + k], xm = sh[b + m - k];
+			double2 B = cmul(make_double2(xk.x - xm.x, xk.y + xm.y),
+					twiddle_at(tw, k << tsh, 1.0));
+			double2 B2 = cmul(make_double2(xm.x - xk.x, xm.y + xk.y),
+					twiddle_at(tw, (m - k) << tsh, 1.0));
+			sh[b + k] = make_double2((xk.x + xm.x) - B.y, (xk.y - xm.y) + B.x);
+			sh[b + m - k] = make_double2((xm.x + xk.x) - B2.y, (xm.y - xk.y) + B2.x);
+		}
+	}
+	__syncthreads();
+	small_fft(sh, stride, 1, lgm, lgny, tw, lgN, +1.0);
+	double2 *__restrict__ phi2 = (double2 *) (a.phi + n0);
+	for(int i = tid; i < m * ny; i += NT)
+		phi2[i] = sh[(i >> lgm) * stride + (i & (m - 1))];
+	if(a.E)
+	{
+		// k_efield's expressions
+		const double *f = (const double *) sh;
+		for(int i = tid; i < n; i += NT)
+		{
+			const int iy = i >> lgnx, ix = i & (nx - 1), row = iy * 2 * stride;
+			const int xm = (ix - 1) & (nx - 1), xp = (ix + 1) & (nx - 1);
+			const int ym = (iy - 1) & (ny - 1), yp = (iy + 1) & (ny - 1);
+			double ey = (f[ym * 2 * stride + ix] - f[yp * 2 * stride + ix]) / dy2;
+			double ex = (f[row + xm] - f[row + xp]) / dx2;
+			if(a.e32)
+				((float2 *) a.E)[n0 + i] = make_float2((float) ex, (float) ey);
+			else
+				((double2 *) a.E)[n0 + i] = make_double2(ex, ey);
+		}
+	}
+	if(a.diag_zero && tid == 0)
+	{
+		DiagSlot *z = &a.diag_zero[diag0 + (iter + 1) % a.ring];
+		z->field = 0.0;
+		z->kinetic = 0.0;
+		z->px = 0.0;
+		z->py = 0.0;
+	}
+}
+
 // E = -grad(phi) (src/field.c:381-406), zeroing of the next rho buffer and
 // of the next diagnostic slot.  Work items: blocks of EF_NODES nodes.
 template <typename T2>
@@ -719,7 +1054,7 @@ fft_lds_attrs(void)
 		(const void *) k_rows_r2c<256>, (const void *) k_rows_c2r<256>, (const void *) k_cols<256>,
 		(const void *) k_rows_r2c<512>, (const void *) k_rows_c2r<512>, (const void *) k_cols<512>,
 		(const void *) k_rows_r2c<1024>, (const void *) k_rows_c2r<1024>,
-		(const void *) k_cols<1024>};
+		(const void *) k_cols<1024>, (const void *) k_solve_small};
 	for(unsigned i = 0; i < sizeof(kern) / sizeof(kern[0]); i++)
 	{
 		hipFuncAttributes fa;
@@ -902,6 +1237,64 @@ cpic_fft_blocking_ok(const Geo *g, int nt_row, int nt_col)
 			hipLaunchKernelGGL(kern<1024>, dim3(grid), dim3(1024), lds, stream, __VA_ARGS__); \
 	} while(0)
 
+// Complex values of a grid's half spectrum, and the LDS of its one-workgroup
+// solve: rows of nx/2 + 1 values, then the cosine tables.
+static int64_t
+small_values(const Geo *g)
+{
+	return (int64_t) (g->nx / 2) * g->ny;
+}
+
+static size_t
+small_lds(const Geo *g)
+{
+	size_t stride = (size_t) g->nx / 2 + 1;
+	return sizeof(double2) * stride * (size_t) g->ny + sizeof(double) * (stride + (size_t) g->ny);
+}
+
+// Whether one workgroup solves the grid (see FFT_SMALL_VALUES).
+static bool
+small_ok(const Geo *g)
+{
+	return small_values(g) <= FFT_SMALL_VALUES && small_lds(g) <= 144 * 1024;
+}
+
+static int
+launch_small(const SmallSolve &a, int P, size_t lds, hipStream_t stream)
+{
+	hipLaunchKernelGGL(k_solve_small, dim3(P), dim3(SMALL_NT), lds, stream, a);
+	HIPCHK(hipGetLastError());
+	return 0;
+}
+
+// Whether every plasma of the batch has the one-workgroup solve.
+int
+cpic_solve_is_small(const cpic_dev *d)
+{
+	for(int p = 0; p < d->P; p++)
+		if(!small_ok(&d->hgeo[p]))
+			return 0;
+	return 1;
+}
+
+static int
+solve_small(cpic_dev *d, SmallSolve &a)
+{
+	size_t lds = 0;
+	for(int p = 0; p < d->P; p++)
+		lds = lds < small_lds(&d->hgeo[p]) ? small_lds(&d->hgeo[p]) : lds;
+	a.geo = d->geo;
+	a.costab = d->costab;
+	a.tw = d->tw;
+	a.lgN = d->lgN;
+	a.ring = d->ring;
+	a.st = d->st;
+	int slot = cpic_kt_begin(d, "solve_small");
+	int ret = launch_small(a, d->P, lds, d->stream);
+	cpic_kt_end(d, slot);
+	return ret;
+}
+
 // phi = S rho for every plasma of the batch (rho and phi laid out like the
 // state's own buffers); with diag, the field energy of each plasma goes to
 // its slot of the current step, with eout, it is added to eout[p].
@@ -913,6 +1306,17 @@ solve(cpic_dev *d, const double *rho, double *phi, DiagSlot *diag, double *rho_z
 	const int P = d->P;
 	const int *pre = d->pre;
 
+	if(d->fft_small)
+	{
+		SmallSolve a = {};
+		a.rho = rho;
+		a.phi = phi;
+		a.diag = diag;
+		a.rho_zero = rho_zero;
+		a.diag_zero = diag_zero;
+		a.eout = eout;
+		return solve_small(d, a);
+	}
 	slot = cpic_kt_begin(d, "fft_rows_r2c");
 	FFT_LAUNCH(k_rows_r2c, d->fft_nt_row, d->rowblocks, d->lds_rows, d->stream,
 			d->geo, pre + PRE_ROW * (P + 1), P, rho, d->ghat, d->tw, d->lgN);
@@ -976,6 +1380,43 @@ cpic_solve_ptr_energy(cpic_dev *d, const double *rho, double *phi, double *rho_z
 		double *energy)
 {
 	return solve(d, rho, phi, (DiagSlot *) NULL, rho_zero, (DiagSlot *) NULL, energy);
+}
+
+// The energy variant with E = -grad phi into E (FP64 or FP32 as the handle's).
+int
+cpic_solve_ptr_E(cpic_dev *d, const double *rho, double *phi, double *rho_zero, double *energy,
+		void *E)
+{
+	int ret;
+	if(d->fft_small)
+	{
+		SmallSolve a = {};
+		a.rho = rho;
+		a.phi = phi;
+		a.rho_zero = rho_zero;
+		a.eout = energy;
+		a.E = E;
+		a.e32 = d->prec == 32;
+		return solve_small(d, a);
+	}
+	if((ret = cpic_solve_ptr_energy(d, rho, phi, rho_zero, energy)))
+		return ret;
+	return cpic_efield_ptr(d, phi, E);
+}
+
+// lrho = S (D^T lE - srho rho), lE_zero = 0, for a handle with the
+// one-workgroup solve and one plasma.
+int
+cpic_solve_transposed_small(cpic_dev *d, const double2 *lE, const double *rho, double srho,
+		double2 *lE_zero, double *lrho)
+{
+	SmallSolve a = {};
+	a.rho = rho;
+	a.phi = lrho;
+	a.lE = lE;
+	a.srho = srho;
+	a.lE_zero = lE_zero;
+	return solve_small(d, a);
 }
 
 int
@@ -1130,6 +1571,19 @@ cpic_solve_xy_noalloc(int64_t nx, int64_t ny, const double *rho, double *phi, vo
 	if(!cpic_fft_blocking_ok(&g, nt_row, nt_col))
 		return CPIC_EINVAL;
 	cpic_fft_spread(&g, 1);
+	unsigned char *ws;
+	if(small_ok(&g))
+	{
+		// one launch, tables included; no workspace
+		SmallSolve a = {};
+		if((ret = ws_get(&ws)))          // raises the kernels' LDS limits
+			return ret;
+		a.one = g;
+		a.rho = rho;
+		a.phi = phi;
+		a.lgN = ilog2(nx > ny ? nx : ny);
+		return launch_small(a, 1, small_lds(&g), (hipStream_t) stream);
+	}
 
 	int64_t hx = nx / 2 + 1, N = nx > ny ? nx : ny;
 	size_t o_cos = WS_TABLES;
@@ -1143,7 +1597,6 @@ cpic_solve_xy_noalloc(int64_t nx, int64_t ny, const double *rho, double *phi, vo
 				need, (size_t) CPIC_NOALLOC_WORKSPACE_BYTES);
 		return CPIC_ESIZE;
 	}
-	unsigned char *ws;
 	if((ret = ws_get(&ws)))
 		return ret;
 
