@@ -389,24 +389,14 @@ static __device__ __forceinline__ int row_block(int b, int n)
 }
 
 // Pass 1: R rows per block of NT threads; row y real of length nx = 2m.
+// Row block rb of one plasma.
 template <int NT>
-__global__ __launch_bounds__(NT, FFT_MIN_WAVES)
-void k_rows_r2c(const Geo *__restrict__ geo, const int *__restrict__ pre, int P,
-		const double *__restrict__ rho_all, double2 *__restrict__ ghat_all,
-		const double2 *__restrict__ tw, int lgN)
+static __device__ __forceinline__ void rows_r2c(double2 *sh, int nx, int lgnx, int ny, int R, int rb,
+		const double *__restrict__ rho, double2 *__restrict__ ghat, const TwRef &twr, int lgN)
 {
-	extern __shared__ double2 sh[];
-	const int rb = blockIdx.x;
-	int p = find_plasma(pre, P, rb);
-	const Geo g = geo[p];
-	int nx = g.nx, ny = g.ny, R = g.R;
-	const double *__restrict__ rho = rho_all + g.node0;
-	double2 *__restrict__ ghat = ghat_all + g.ghat0;
-	int m = nx >> 1, lgm = g.lgnx - 1;
+	int m = nx >> 1, lgm = lgnx - 1;
 	int stride = m + 1;
-	int y0 = (rb - pre[p]) * R;
-	__shared__ TwLds s_tw;
-	const TwRef twr = tw_fill(s_tw, tw, lgN);
+	int y0 = rb * R;
 
 	// the first stage reads the rows straight from rho (as complex pairs)
 	const double2 *__restrict__ rows2 = (const double2 *) (rho + (int64_t) y0 * nx);
@@ -449,6 +439,22 @@ void k_rows_r2c(const Geo *__restrict__ geo, const int *__restrict__ pre, int P,
 		if(2 * k != m)
 			ghat[(int64_t) (m - k) * ny + y0 + r] = xm;
 	}
+}
+
+template <int NT>
+__global__ __launch_bounds__(NT, FFT_MIN_WAVES)
+void k_rows_r2c(const Geo *__restrict__ geo, const int *__restrict__ pre, int P,
+		const double *__restrict__ rho_all, double2 *__restrict__ ghat_all,
+		const double2 *__restrict__ tw, int lgN)
+{
+	extern __shared__ double2 sh[];
+	__shared__ TwLds s_tw;
+	const int rb = blockIdx.x;
+	int p = find_plasma(pre, P, rb);
+	const Geo g = geo[p];
+	const TwRef twr = tw_fill(s_tw, tw, lgN);
+	rows_r2c<NT>(sh, g.nx, g.lgnx, g.ny, g.R, rb - pre[p], rho_all + g.node0, ghat_all + g.ghat0,
+			twr, lgN);
 }
 
 // Pass 2: C columns (kx) per block of NT threads, each ny long and contiguous.
@@ -1012,6 +1018,11 @@ void k_efield(const Geo *__restrict__ geo, const int *__restrict__ pre, int P,
 	}
 }
 
+template <int NT>
+__global__ void k_noalloc_rows(Geo g, int rows, int cols, int lgN, unsigned char *__restrict__ ws,
+		double *__restrict__ costab, double2 *__restrict__ tw, const double *__restrict__ rho,
+		double2 *__restrict__ ghat);
+
 // ---------------------------------------------------------------- host ---
 
 // exp(+2 pi i k/n), 0 <= k <= n/2, by octant reduction so that the
@@ -1047,14 +1058,15 @@ twiddle(int64_t k, int64_t n, double *c, double *s)
 // One row of 8192 points needs 64 KB + 16 B of LDS, a column 128 KB: the
 // passes' dynamic LDS limit is raised, leaving room for each kernel's
 // static LDS.
+#define FFT_KERNELS(nt) (const void *) k_rows_r2c<nt>, (const void *) k_rows_c2r<nt>, \
+	(const void *) k_cols<nt>, (const void *) k_noalloc_rows<nt>
+
 static int
 fft_lds_attrs(void)
 {
 	const void *kern[] = {
-		(const void *) k_rows_r2c<256>, (const void *) k_rows_c2r<256>, (const void *) k_cols<256>,
-		(const void *) k_rows_r2c<512>, (const void *) k_rows_c2r<512>, (const void *) k_cols<512>,
-		(const void *) k_rows_r2c<1024>, (const void *) k_rows_c2r<1024>,
-		(const void *) k_cols<1024>, (const void *) k_solve_small};
+		FFT_KERNELS(256), FFT_KERNELS(512), FFT_KERNELS(1024),
+		(const void *) k_solve_small};
 	for(unsigned i = 0; i < sizeof(kern) / sizeof(kern[0]); i++)
 	{
 		hipFuncAttributes fa;
@@ -1516,6 +1528,51 @@ void k_noalloc_setup(Geo g, int rows, int cols, int lgN, unsigned char *__restri
 		twiddle(k, N, &tw[k].x, &tw[k].y);
 }
 
+// The same by the first pass itself: every block makes the twiddles that it needs, so
+// nothing has to be there before it, and its share of the tables for the
+// other passes.  The sines and cosines are the last wavefronts' work, which
+// have few butterflies in the first stage, so that the others' loads of
+// rho go out meanwhile.  For up to NOALLOC_FOLD row blocks (one per CU) that takes less
+// than the set-up launch it saves: allocation-free solve at 256^2 20.5 ->
+// 18.3 us, 512^2 22.2 -> 20.4, 1024x128 21.4 -> 20.2, 1024^2 36.8 -> 34.5; with more
+// the blocks' own tables cost more: 2048^2 (512 blocks) 64.8 -> 70.2.
+#define NOALLOC_FOLD 256
+template <int NT>
+__global__ __launch_bounds__(NT, FFT_MIN_WAVES)
+void k_noalloc_rows(Geo g, int rows, int cols, int lgN, unsigned char *__restrict__ ws,
+		double *__restrict__ costab, double2 *__restrict__ tw, const double *__restrict__ rho,
+		double2 *__restrict__ ghat)
+{
+	extern __shared__ double2 sh[];
+	__shared__ TwLds s_tw;
+	const int back = NT - 1 - (int) threadIdx.x;
+	if(blockIdx.x == 0 && threadIdx.x == 0)
+	{
+		*(Geo *) (ws + WS_GEO) = g;
+		int *pre = (int *) (ws + WS_PRE);
+		pre[0] = 0;
+		pre[1] = rows;
+		pre[2] = 0;
+		pre[3] = cols;
+		StepState *st = (StepState *) (ws + WS_STEP);
+		st->iter = -1;
+	}
+	const TwRef twr = tw_make(s_tw, lgN, back);
+	// the workspace's tables, dealt out over the blocks; wavefronts before
+	// those of the block's own table
+	const int hx = g.nx / 2 + 1, ncos = hx + g.ny, N = 1 << lgN;
+	const double cx = 2.0 * M_PI / g.nx, cy = 2.0 * M_PI / g.ny;
+	for(int k = blockIdx.x + gridDim.x * ((back + NT - 128) & (NT - 1)); k < ncos + N / 2 + 1;
+			k += gridDim.x * NT)
+	{
+		if(k < ncos)
+			costab[k] = k < hx ? cos(cx * k) : cos(cy * (k - hx));
+		else
+			twiddle(k - ncos, N, &tw[k - ncos].x, &tw[k - ncos].y);
+	}
+	rows_r2c<NT>(sh, g.nx, g.lgnx, g.ny, g.R, blockIdx.x, rho, ghat, twr, lgN);
+}
+
 // Device address of this GPU's workspace (the current device), looked up
 // on the first call on each GPU.
 static int
@@ -1611,17 +1668,26 @@ cpic_solve_xy_noalloc(int64_t nx, int64_t ny, const double *rho, double *phi, vo
 	double *costab = (double *) (ws + o_cos);
 	double2 *tw = (double2 *) (ws + o_tw);
 	double2 *ghat = (double2 *) (ws + o_ghat);
-	int64_t nset = hx > ny ? hx : ny;
-	if(N / 2 + 1 > nset)
-		nset = N / 2 + 1;
-	nset = (nset + CPIC_BLOCK - 1) / CPIC_BLOCK;
 
-	hipLaunchKernelGGL(k_noalloc_setup, dim3((unsigned) nset), dim3(CPIC_BLOCK), 0, s, g,
-			rows, cols, lgN, ws, costab, tw);
-	HIPCHK(hipGetLastError());
-	FFT_LAUNCH(k_rows_r2c, nt_row, rows, lds_rows, s,
-			geo, pre, 1, rho, ghat, (const double2 *) tw, lgN);
-	HIPCHK(hipGetLastError());
+	if(rows <= NOALLOC_FOLD)
+	{
+		FFT_LAUNCH(k_noalloc_rows, nt_row, rows, lds_rows, s,
+				g, rows, cols, lgN, ws, costab, tw, rho, ghat);
+		HIPCHK(hipGetLastError());
+	}
+	else
+	{
+		int64_t nset = hx > ny ? hx : ny;
+		if(N / 2 + 1 > nset)
+			nset = N / 2 + 1;
+		nset = (nset + CPIC_BLOCK - 1) / CPIC_BLOCK;
+		hipLaunchKernelGGL(k_noalloc_setup, dim3((unsigned) nset), dim3(CPIC_BLOCK), 0, s, g,
+				rows, cols, lgN, ws, costab, tw);
+		HIPCHK(hipGetLastError());
+		FFT_LAUNCH(k_rows_r2c, nt_row, rows, lds_rows, s,
+				geo, pre, 1, rho, ghat, (const double2 *) tw, lgN);
+		HIPCHK(hipGetLastError());
+	}
 	FFT_LAUNCH(k_cols, nt_col, cols, lds_cols, s,
 			geo, pre + 2, 1, ghat, (const double *) costab, (const double2 *) tw, lgN,
 			(DiagSlot *) NULL, 1, st, (double *) NULL);
