@@ -329,6 +329,21 @@ void k_adj_push(Geo g, AdjSpecies k, int set_r, double dtp, int64_t n,
 	int64_t p0 = (int64_t) blockIdx.x * (PPT * CPIC_BLOCK);
 	int ix[PPT], iy[PPT];
 	double rx[PPT], ry[PPT];
+	// all of the thread's loads first, unconditional: behind a bounds check, or
+	// behind the stores of the particle before (which the compiler cannot tell
+	// from the positions), each particle's were waited for in turn
+	double lpx[PPT], lpy[PPT], lux[PPT], luy[PPT];
+	int ls[PPT];
+#pragma unroll
+	for(int u = 0; u < PPT; u++)
+	{
+		const int64_t i = min(p0 + u * CPIC_BLOCK + (int) threadIdx.x, n - 1);
+		lpx[u] = x[i];
+		lpy[u] = y[i];
+		lux[u] = ux[i];
+		luy[u] = uy[i];
+		ls[u] = sp[i];
+	}
 #pragma unroll
 	for(int u = 0; u < PPT; u++)
 	{
@@ -336,10 +351,10 @@ void k_adj_push(Geo g, AdjSpecies k, int set_r, double dtp, int64_t n,
 		ix[u] = -1;
 		if(i >= n)
 			continue;
-		int s = sp[i];
+		const int s = ls[u];
 		int jx, jy;
 		double qx, qy;
-		double px = x[i], py = y[i];
+		double px = lpx[u], py = lpy[u];
 		cell_of(g, px, py, jx, jy, qx, qy);
 		int j1x = jx + 1 == g.nx ? 0 : jx + 1;
 		int j1y = jy + 1 == g.ny ? 0 : jy + 1;
@@ -355,7 +370,7 @@ void k_adj_push(Geo g, AdjSpecies k, int set_r, double dtp, int64_t n,
 		ey = fma(w01, e01.y, ey);
 		ey = fma(w10, e10.y, ey);
 		ey = fma(w11, e11.y, ey);
-		double uu = ux[i], vv = uy[i];
+		double uu = lux[u], vv = luy[u];
 		boris_bz<double>(k.h[s], k.tz[s], k.sz[s], ex, ey, uu, vv);
 		if(fabs(uu) > g.umax_x || fabs(vv) > g.umax_y)
 			bad = true;
@@ -385,11 +400,8 @@ void k_adj_push(Geo g, AdjSpecies k, int set_r, double dtp, int64_t n,
 	box_zero(b, sacc, 1);
 #pragma unroll
 	for(int u = 0; u < PPT; u++)
-	{
-		int64_t i = p0 + u * CPIC_BLOCK + threadIdx.x;
 		if(ix[u] >= 0)
-			dep1(g, b, sacc, rho_next, ix[u], iy[u], rx[u], ry[u], k.c[sp[i]]);
-	}
+			dep1(g, b, sacc, rho_next, ix[u], iy[u], rx[u], ry[u], k.c[ls[u]]);
 	box_flush(g, b, sacc, 1, rho_next, 1);
 }
 
