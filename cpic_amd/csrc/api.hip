@@ -523,41 +523,53 @@ cpic_dev_destroy(cpic_dev_t *d)
 // ---------------------------------------------------------- downloads ---
 
 // Copies device ranges to ordinary host memory after the work queued on the
-// handle's stream, or (up) the other way.  Copying straight into pageable memory runs at ~9 GB/s:
-// the runtime's own staging is one thread's, and for a fresh destination
-// that thread also takes every page fault.  Here the ranges go, DL_CHUNK
-// bytes at a time, through two pinned buffers; while one is filled by DMA,
+// handle's stream, or (up) the other way.  Copying straight into pageable
+// memory runs at ~9 GB/s: the runtime's own staging is one thread's, and for a
+// fresh destination that thread also takes every page fault.  Here the ranges
+// go through two pinned buffers, a chunk at a time; while one is filled by DMA,
 // the threads copy the other out, each taking its share of the chunk's pages
-// (and faults).  Small downloads copy on the calling thread: starting threads
-// would cost more than they save.
+// (and faults).  Small copies run on the calling thread: starting threads
+// would cost more than they save.  Pinning costs ~0.1 ms per MB, once per
+// handle, so a handle that never copies more than 2 DL_CHUNK at once has
+// small buffers.
 static int
 copy_ranges(cpic_dev *d, int nr, const DlRange *r, bool up)
 {
 	struct Piece { size_t at, off, bytes; int range; };
 	std::vector<Piece> pieces;
 	std::vector<size_t> first;         // pieces of chunk c: [first[c], first[c+1])
-	size_t total = 0, fill = DL_CHUNK;
-	if(!d->pin && hipHostMalloc((void **) &d->pin, 2 * DL_CHUNK, hipHostMallocDefault)
-			!= hipSuccess)
+	size_t total = 0;
+	for(int k = 0; k < nr; k++)
+		total += r[k].bytes;
+	const size_t want = total > 2 * DL_CHUNK ? DL_CHUNK : DL_CHUNK_SMALL;
+	if(d->pinchunk < want)
 	{
-		d->pin = NULL;
-		return CPIC_ENOMEM;
+		if(d->pin)
+			hipHostFree(d->pin);
+		d->pinchunk = 0;
+		if(hipHostMalloc((void **) &d->pin, 2 * want, hipHostMallocDefault) != hipSuccess)
+		{
+			d->pin = NULL;
+			return CPIC_ENOMEM;
+		}
+		d->pinchunk = want;
 	}
+	const size_t chunk = d->pinchunk;
+	size_t fill = chunk;
 	try
 	{
 		for(int k = 0; k < nr; k++)
 			for(size_t o = 0; o < r[k].bytes; )
 			{
-				if(fill == DL_CHUNK)
+				if(fill == chunk)
 				{
 					first.push_back(pieces.size());
 					fill = 0;
 				}
-				size_t n = std::min(DL_CHUNK - fill, r[k].bytes - o);
+				size_t n = std::min(chunk - fill, r[k].bytes - o);
 				pieces.push_back({fill, o, n, k});
 				fill += n;
 				o += n;
-				total += n;
 			}
 		first.push_back(pieces.size());
 	}
@@ -572,7 +584,7 @@ copy_ranges(cpic_dev *d, int nr, const DlRange *r, bool up)
 	int workers = 0;
 	// thread t of n copies its share of every piece of chunk c
 	auto copy = [&](int c, int t, int n) {
-		char *b = d->pin + (size_t) (c & 1) * DL_CHUNK;
+		char *b = d->pin + (size_t) (c & 1) * chunk;
 		for(size_t k = first[c]; k < first[c + 1]; k++)
 		{
 			const Piece &p = pieces[k];
@@ -587,7 +599,7 @@ copy_ranges(cpic_dev *d, int nr, const DlRange *r, bool up)
 	};
 	// queues the DMA of chunk c
 	auto dma = [&](int c) -> hipError_t {
-		char *b = d->pin + (size_t) (c & 1) * DL_CHUNK;
+		char *b = d->pin + (size_t) (c & 1) * chunk;
 		hipError_t e = hipSuccess;
 		for(size_t k = first[c]; k < first[c + 1] && e == hipSuccess; k++)
 		{

@@ -42,7 +42,8 @@
 #define CPIC_MARGIN 1            // cells of drift covered by the LDS tile regions
 #define CPIC_BUCKET_MAX (1 << 27) // slots of one (tile, species) bucket: 32-bit byte offsets
 #define CPIC_MAX_KERNELS 24
-#define DL_CHUNK ((size_t) 4 << 20)      // bytes of a download's bounce buffer
+#define DL_CHUNK ((size_t) 4 << 20)      // bytes of a bounce buffer for host copies
+#define DL_CHUNK_SMALL ((size_t) 512 << 10)   // the same while no copy has exceeded 2 DL_CHUNK
 #define DL_KEEP ((size_t) 256 << 20)     // largest download workspace a handle keeps
 
 // device error word bits
@@ -243,9 +244,10 @@ struct cpic_dev {
 	int graph_ok;
 	int capturing;           // inside hipStreamBeginCapture/EndCapture
 
-	// host copies: pinned bounce buffers (2 x DL_CHUNK bytes) and the particle
+	// host copies: pinned bounce buffers (2 x pinchunk bytes) and the particle
 	// downloads' device workspace, both kept between calls
 	char *pin;
+	size_t pinchunk;
 	char *dl;
 	size_t dlcap;
 
