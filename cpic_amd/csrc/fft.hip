@@ -36,6 +36,7 @@
 // plasmas of a batch: block b takes the b-th item of the pass's work list
 // (row block or column block) and finds its plasma by binary search.
 #include "dev.h"
+#include "picmath.h"
 
 #include <math.h>
 #include <pthread.h>
@@ -771,6 +772,7 @@ void k_solve_small(SmallSolve a)
 	const int64_t n0 = plan ? gp->node0 : 0;
 	const int diag0 = plan ? gp->diag0 : 0;
 	const double dx2 = plan ? 2 * gp->dx : 0.0, dy2 = plan ? 2 * gp->dy : 0.0;
+	const double rx2 = 1.0 / dx2, ry2 = 1.0 / dy2;
 	const double invN = 1.0 / ((double) nx * (double) ny);
 	double *cosx = (double *) (sh + stride * ny), *cosy = cosx + stride;
 	const long long iter = a.st ? a.st->iter : -1;
@@ -807,24 +809,26 @@ void k_solve_small(SmallSolve a)
 		// D^T lE - srho rho (the transpose of the E stencil), and the other
 		// lE buffer zeroed
 		// two neighbouring nodes i, i + 1 per value
+		with_div(dx2, dy2, [&](auto div) {
 #pragma unroll
-		for(int v = 0; v < 2; v++)
-		{
-			const int i = 2 * (tid + v * NT);
-			if(i >= n)
-				continue;
-			const int iy = i >> lgnx, ix = i & (nx - 1), row = iy << lgnx;
-			const int ym = ((iy - 1) & (ny - 1)) << lgnx, yp = ((iy + 1) & (ny - 1)) << lgnx;
-			auto psi = [&](int x, double r) {
-				const int xm = (x - 1) & (nx - 1), xp = (x + 1) & (nx - 1);
-				double lphi = (a.lE[row + xp].x - a.lE[row + xm].x) / dx2 +
-					(a.lE[yp + x].y - a.lE[ym + x].y) / dy2;
-				return lphi - a.srho * r;
-			};
-			in[v] = make_double2(psi(ix, in[v].x), psi(ix + 1, in[v].y));
-			a.lE_zero[i] = make_double2(0.0, 0.0);
-			a.lE_zero[i + 1] = make_double2(0.0, 0.0);
-		}
+			for(int v = 0; v < 2; v++)
+			{
+				const int i = 2 * (tid + v * NT);
+				if(i >= n)
+					continue;
+				const int iy = i >> lgnx, ix = i & (nx - 1), row = iy << lgnx;
+				const int ym = ((iy - 1) & (ny - 1)) << lgnx, yp = ((iy + 1) & (ny - 1)) << lgnx;
+				auto psi = [&](int x, double r) {
+					const int xm = (x - 1) & (nx - 1), xp = (x + 1) & (nx - 1);
+					double lphi = div(a.lE[row + xp].x - a.lE[row + xm].x, dx2, rx2) +
+						div(a.lE[yp + x].y - a.lE[ym + x].y, dy2, ry2);
+					return lphi - a.srho * r;
+				};
+				in[v] = make_double2(psi(ix, in[v].x), psi(ix + 1, in[v].y));
+				a.lE_zero[i] = make_double2(0.0, 0.0);
+				a.lE_zero[i + 1] = make_double2(0.0, 0.0);
+			}
+		});
 	}
 #pragma unroll
 	for(int v = 0; v < 2; v++)
@@ -951,18 +955,20 @@ void k_solve_small(SmallSolve a)
 	{
 		// k_efield's expressions
 		const double *f = (const double *) sh;
-		for(int i = tid; i < n; i += NT)
-		{
-			const int iy = i >> lgnx, ix = i & (nx - 1), row = iy * 2 * stride;
-			const int xm = (ix - 1) & (nx - 1), xp = (ix + 1) & (nx - 1);
-			const int ym = (iy - 1) & (ny - 1), yp = (iy + 1) & (ny - 1);
-			double ey = (f[ym * 2 * stride + ix] - f[yp * 2 * stride + ix]) / dy2;
-			double ex = (f[row + xm] - f[row + xp]) / dx2;
-			if(a.e32)
-				((float2 *) a.E)[n0 + i] = make_float2((float) ex, (float) ey);
-			else
-				((double2 *) a.E)[n0 + i] = make_double2(ex, ey);
-		}
+		with_div(dx2, dy2, [&](auto div) {
+			for(int i = tid; i < n; i += NT)
+			{
+				const int iy = i >> lgnx, ix = i & (nx - 1), row = iy * 2 * stride;
+				const int xm = (ix - 1) & (nx - 1), xp = (ix + 1) & (nx - 1);
+				const int ym = (iy - 1) & (ny - 1), yp = (iy + 1) & (ny - 1);
+				double ey = div(f[ym * 2 * stride + ix] - f[yp * 2 * stride + ix], dy2, ry2);
+				double ex = div(f[row + xm] - f[row + xp], dx2, rx2);
+				if(a.e32)
+					((float2 *) a.E)[n0 + i] = make_float2((float) ex, (float) ey);
+				else
+					((double2 *) a.E)[n0 + i] = make_double2(ex, ey);
+			}
+		});
 	}
 	if(a.diag_zero && tid == 0)
 	{

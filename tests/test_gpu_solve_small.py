@@ -86,6 +86,31 @@ def test_gradient_matches_the_torch_reference(nx, ny, n):
     run.close()
 
 
+@pytest.mark.parametrize("dx,dy", [(1.0, 1.0), (0.25, 0.25), (0.3, 0.3), (0.3, 0.25), (0.25, 0.3)])
+def test_gradient_with_cells_of_other_sizes(dx, dy):
+    """Cell sizes whose E stencil divides and whose multiplies; bounds as above."""
+    from cpic_amd import diff
+    from common import rel_l2
+    from torch_pic import TorchPIC
+    n, nx, ny = 700, 32, 16
+    L = (nx * dx, ny * dy)
+    r = np.random.default_rng(9)
+    st = [r.random(n) * L[0], r.random(n) * L[1], r.normal(0, 0.02 * dx, n),
+          r.normal(0, 0.02 * dy, n)]
+    sp = np.zeros(n, np.int32)
+    run = diff.AdjointRun(nx, ny, L, 0.1, [-1.0], [n / (nx * ny)], sp)
+    ref = TorchPIC(nx, ny, L, 0.1, [-1.0], [n / (nx * ny)])
+    loss, _ = run.forward(*st, 4, 2)
+    g = run.backward(1.0)
+    t = [torch.tensor(a, requires_grad=True) for a in st]
+    lref, _ = ref.run(*t, sp, 4)
+    lref.backward()
+    assert abs(loss - float(lref.detach())) <= 1e-10 * abs(float(lref.detach()))
+    for a, b in zip(g, t):
+        assert rel_l2(a, b.grad.numpy()) < 1e-7
+    run.close()
+
+
 def test_batch_of_small_grids_of_different_shapes():
     shapes = [(64, 64), (16, 32), (128, 32), (8, 8)]
     b = ca.Batch([ca.make_desc(nx, ny, (nx, ny), 0.1, [-1.0], [1.0]) for nx, ny in shapes])
