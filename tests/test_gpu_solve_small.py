@@ -47,7 +47,7 @@ def test_solve_matches_the_spectral_reference(nx, ny):
     ref = reference(rho)
     tol = 1e-15 * max(nx, ny) ** 2 + 1e-13
     assert np.abs(noalloc(rho) - ref).max() <= tol * np.abs(ref).max()
-    # the handle's solve and the E stencil, a batch of two with one empty
+    # the handle's solve, and the E array made from its phi
     d = ca.Device(nx, ny, (nx, ny), 0.1, [-1.0], [1.0])
     d.set_field("rho", rho)
     d.stage("field_E", 0)
