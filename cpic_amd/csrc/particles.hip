@@ -1697,8 +1697,13 @@ void k_id_range(Geo g, Buckets bk, int par, Parts p, int s, DlInfo *__restrict__
 }
 
 // The species as arrays (x, y, ux, uy, Ex, Ey, index, cell, n elements each):
-// in storage order, or with `seen` (n bits, zero) particle i at position
+// in storage order (tile by tile, slot by slot, holes left out), or with
+// `seen` (n bits, zero) particle i at position
 // i - info->lo, which the caller has found to be below n for all of them.
+// A particle's place in storage order is counted, not claimed, so that a state
+// gives the same rows in every call: the used slots of the rounds before,
+// of the wavefronts before in this round (one line of s_used, the lines
+// taking turns, so that one barrier per round does) and of the lanes before.
 template <typename T, bool IDS, bool PE>
 __global__ __launch_bounds__(CPIC_BLOCK)
 void k_download(Geo g, Buckets bk, int par, Parts p, int s, const int64_t *__restrict__ off,
@@ -1712,28 +1717,45 @@ void k_download(Geo g, Buckets bk, int par, Parts p, int s, const int64_t *__res
 	const BucketNow v = bucket_now(bk, par, b);
 	int64_t *__restrict__ oid = (int64_t *) (out + 6 * n), *__restrict__ ocell = oid + n;
 	const long long lo = seen ? info->lo : 0;
-	__shared__ int s_done;
-	if(threadIdx.x == 0)
-		s_done = 0;
-	__syncthreads();
-	for(int j = threadIdx.x; j < v.n; j += blockDim.x)
+	__shared__ int s_used[2][CPIC_BLOCK / 64];
+	const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+	int64_t next = seen ? 0 : off[tile];
+	for(int j0 = 0, turn = 0; j0 < v.n; j0 += CPIC_BLOCK, turn ^= 1)
 	{
-		int64_t slot = bk.start[b] + j;
+		const int j = j0 + (int) threadIdx.x;
+		const int64_t slot = bk.start[b] + j;
 		PState<T> q;
-		load_p<T>(p, slot, q, IDS);
-		if(!slot_used(v, j, q.x))
-			continue;
-		int64_t o;
+		bool used = false;
+		if(j < v.n)
+		{
+			load_p<T>(p, slot, q, IDS);
+			used = slot_used(v, j, q.x);
+		}
+		int64_t o = -1;
 		if(IDS && seen)
 		{
-			o = q.id - lo;
-			unsigned bit = 1u << (o & 31);
-			if(o >= 0 && o < n && (atomicOr(&seen[o >> 5], bit) & bit))
-				info->dup = 1;
+			if(used)
+			{
+				o = q.id - lo;
+				unsigned bit = 1u << (o & 31);
+				if(o >= 0 && o < n && (atomicOr(&seen[o >> 5], bit) & bit))
+					info->dup = 1;
+			}
 		}
 		else
-			o = off[tile] + atomicAdd(&s_done, 1);
-		if(o < 0 || o >= n)
+		{
+			const unsigned long long mask = __ballot(used);
+			if(lane == 0)
+				s_used[turn][wid] = __popcll(mask);
+			__syncthreads();
+			o = next + lanes_below(mask);
+			for(int w = 0; w < CPIC_BLOCK / 64; w++)
+			{
+				o += w < wid ? s_used[turn][w] : 0;
+				next += s_used[turn][w];
+			}
+		}
+		if(!used || o < 0 || o >= n)
 			continue;
 		T x = q.x, y = q.y;
 		CellPos c;
