@@ -956,6 +956,15 @@ grow(double **p, int64_t *cap, int64_t want)
 	return 0;
 }
 
+static void
+release(double **p, int64_t *cap)
+{
+	if(*p)
+		hipFree(*p);
+	*p = NULL;
+	*cap = 0;
+}
+
 static int
 zero(cpic_adj *a, double *p, int64_t n)
 {
@@ -1123,25 +1132,30 @@ download_unsorted(cpic_adj *a, double *const *src, double *const *dst)
 }
 
 // Whether this forward keeps its position history, whose memory is then there.
+// The buffers of the way not taken, left by an earlier forward, are given back.
 static bool
 pos_history(cpic_adj *a, int64_t nsteps)
 {
 	size_t avail = 0, total = 0;
-	double want = 2.0 * (double) a->n * (double) nsteps;
-	if(a->phist_off || want * sizeof(double) > (double) ADJ_POS_HISTORY_MAX)
-		return false;
-	if((double) a->phcap >= want)
-		return true;
-	if(hipMemGetInfo(&avail, &total) != hipSuccess ||
-			want * sizeof(double) > 0.5 * ((double) avail + 8.0 * (double) a->phcap))
+	const double want = 2.0 * (double) a->n * (double) nsteps;
+	const double held = (double) a->phcap + (double) a->ckcap + (double) a->segcap;
+	bool keep = a->fhist && !a->phist_off && want * sizeof(double) <= (double) ADJ_POS_HISTORY_MAX;
+	if(keep && (double) a->phcap < want)
+		keep = hipMemGetInfo(&avail, &total) == hipSuccess &&
+			want * sizeof(double) <= 0.5 * ((double) avail + sizeof(double) * held);
+	if(keep)
 	{
-		(void) hipGetLastError();
-		return false;
+		release(&a->ck, &a->ckcap);
+		release(&a->seg, &a->segcap);
+		keep = !grow(&a->ph, &a->phcap, (int64_t) want);
 	}
-	if(!grow(&a->ph, &a->phcap, (int64_t) want))
-		return true;
-	(void) hipGetLastError();   // no room: checkpoints instead
-	return false;
+	if(!keep)
+	{
+		// checkpoints instead
+		(void) hipGetLastError();
+		release(&a->ph, &a->phcap);
+	}
+	return keep;
 }
 
 extern "C" int
@@ -1178,7 +1192,7 @@ cpic_adj_forward(cpic_adj_t *a, const double *x, const double *y, const double *
 		else
 			(void) hipGetLastError();   // no room: the reverse recomputes instead
 	}
-	a->phist = a->fhist && pos_history(a, nsteps);
+	a->phist = pos_history(a, nsteps);
 	if(!a->phist && (ret = grow(&a->ck, &a->ckcap, 4 * n * nck)))
 		return ret;
 	HIPCHK(hipEventRecord(a->ev[0], a->d->stream));

@@ -308,8 +308,9 @@ int cpic_adj_device_ms(cpic_adj_t *adj, double *forward_ms, double *backward_ms)
 int cpic_adj_set_field_history(cpic_adj_t *adj, int on);
 
 /* The same for the positions: on = 0 makes later forwards checkpoint every
- * `checkpoint_every` iterations instead (less memory); on = 1 (the default):
- * keep them with the fields when they fit. */
+ * `checkpoint_every` iterations instead (less memory; the next forward gives
+ * the history's back); on = 1 (the default): keep them with the fields when
+ * they fit.  A backward of the forward before the call is not affected. */
 int cpic_adj_set_position_history(cpic_adj_t *adj, int on);
 
 #ifdef __cplusplus
