@@ -17,7 +17,10 @@
 #include "dev.h"
 #include "host_sort.h"
 
+#include <chrono>
 #include <cmath>
+#include <condition_variable>
+#include <mutex>
 #include <stdlib.h>
 #include <string.h>
 
@@ -528,10 +531,13 @@ cpic_dev_destroy(cpic_dev_t *d)
 // fresh destination that thread also takes every page fault.  Here the ranges
 // go through two pinned buffers, a chunk at a time; while one is filled by DMA,
 // the threads copy the other out, each taking its share of the chunk's pages
-// (and faults).  Small copies run on the calling thread: starting threads
-// would cost more than they save.  Pinning costs ~0.1 ms per MB, once per
+// (and faults).  Threads that wait for the first chunk poll for COPY_POLL_US, which
+// covers a device that is idle or nearly so, and then sleep: behind a queue
+// of 0.46 s sixteen of them took 7.1 s of CPU time.  Small copies run on the calling
+// thread: starting threads would cost more than they save.  Pinning costs ~0.1 ms per MB, once per
 // handle, so a handle that never copies more than 2 DL_CHUNK at once has
 // small buffers.
+#define COPY_POLL_US 500
 static int
 copy_ranges(cpic_dev *d, int nr, const DlRange *r, bool up)
 {
@@ -580,6 +586,8 @@ copy_ranges(cpic_dev *d, int nr, const DlRange *r, bool up)
 	const int nchunks = (int) first.size() - 1;
 	const int nt = host_threads((int64_t) total, (int64_t) 1 << 20);
 	std::atomic<int> ready(0), fail(0);
+	std::mutex wake_lock;
+	std::condition_variable wake;
 	std::atomic<int> done[2] = {{0}, {0}};      // shares copied out of each buffer
 	int workers = 0;
 	// thread t of n copies its share of every piece of chunk c
@@ -622,6 +630,30 @@ copy_ranges(cpic_dev *d, int nr, const DlRange *r, bool up)
 		while(done[c & 1].load(std::memory_order_acquire) < workers * (c / 2 + 1))
 			std::this_thread::yield();
 	};
+	// the first chunk's arrival or the failure, to threads that may sleep
+	auto announce = [&](std::atomic<int> &what, int value) {
+		{
+			std::lock_guard<std::mutex> hold(wake_lock);
+			what.store(value, std::memory_order_release);
+		}
+		wake.notify_all();
+	};
+	auto wait_first = [&]() {
+		auto begun = [&]() {
+			return ready.load(std::memory_order_acquire) > 0 || fail.load(std::memory_order_relaxed);
+		};
+		const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(COPY_POLL_US);
+		while(!begun())
+		{
+			if(std::chrono::steady_clock::now() > until)
+			{
+				std::unique_lock<std::mutex> hold(wake_lock);
+				wake.wait(hold, begun);
+				return;
+			}
+			std::this_thread::yield();
+		}
+	};
 	std::vector<std::thread> th;
 	try
 	{
@@ -629,6 +661,7 @@ copy_ranges(cpic_dev *d, int nr, const DlRange *r, bool up)
 		for(int t = 0; nt > 1 && t < nt; t++)
 		{
 			th.emplace_back([&, t]() {
+				wait_first();
 				for(int c = 0; c < nchunks; c++)
 				{
 					while(ready.load(std::memory_order_acquire) <= c)
@@ -652,7 +685,7 @@ copy_ranges(cpic_dev *d, int nr, const DlRange *r, bool up)
 	if(up)
 	{
 		// a chunk's DMA runs while the next one's shares are copied in
-		ready.store(2, std::memory_order_release);
+		announce(ready, 2);
 		for(int c = 0; c < nchunks && e == hipSuccess; c++)
 		{
 			finish(c);
@@ -673,11 +706,14 @@ copy_ranges(cpic_dev *d, int nr, const DlRange *r, bool up)
 				wait_done(c - 2);
 			if((e = dma(c)) != hipSuccess || (e = hipStreamSynchronize(d->stream)) != hipSuccess)
 				break;
-			ready.store(c + 1, std::memory_order_release);
+			if(c == 0)
+				announce(ready, 1);
+			else
+				ready.store(c + 1, std::memory_order_release);
 			finish(c);
 		}
 	if(e != hipSuccess)
-		fail = 1;
+		announce(fail, 1);
 	for(auto &x : th)
 		x.join();
 	if(e != hipSuccess)
