@@ -93,7 +93,7 @@ static __device__ __forceinline__ TwRef tw_fill(TwLds &t, const double2 *__restr
 	return r;
 }
 
-static __host__ __device__ void twiddle(int64_t k, int64_t n, double *c, double *s);
+static __host__ __device__ __forceinline__ void twiddle(int64_t k, int64_t n, double *c, double *s);
 
 // The same tables computed instead of copied, entry k by thread t = k mod the
 // block size.
@@ -450,11 +450,12 @@ void k_rows_r2c(const Geo *__restrict__ geo, const int *__restrict__ pre, int P,
 {
 	extern __shared__ double2 sh[];
 	__shared__ TwLds s_tw;
-	const int rb = blockIdx.x;
-	int p = find_plasma(pre, P, rb);
+	int p = find_plasma(pre, P, blockIdx.x);
 	const Geo g = geo[p];
+	// read before the tables are copied: after them, the loads of rho wait for it
+	const int rb = blockIdx.x - pre[p];
 	const TwRef twr = tw_fill(s_tw, tw, lgN);
-	rows_r2c<NT>(sh, g.nx, g.lgnx, g.ny, g.R, rb - pre[p], rho_all + g.node0, ghat_all + g.ghat0,
+	rows_r2c<NT>(sh, g.nx, g.lgnx, g.ny, g.R, rb, rho_all + g.node0, ghat_all + g.ghat0,
 			twr, lgN);
 }
 
@@ -1033,8 +1034,11 @@ __global__ void k_noalloc_rows(Geo g, int rows, int cols, int lgN, unsigned char
 
 // exp(+2 pi i k/n), 0 <= k <= n/2, by octant reduction so that the
 // quarter points are exact (host tables; the allocation-free solve builds
-// its table on the device with the same reduction)
-static __host__ __device__ void
+// its table on the device with the same reduction).  Always inline: with calls,
+// which the compiler makes of the sines and cosines once several kernels
+// use them, the solve takes 47.6 instead of 46.2 us at 2048x1024 and 20.2
+// instead of 19.7 at 1024x128 (34.3 instead of 34.4 at 1024^2).
+static __host__ __device__ __forceinline__ void
 twiddle(int64_t k, int64_t n, double *c, double *s)
 {
 	int64_t k8 = 8 * k;
@@ -1540,7 +1544,7 @@ void k_noalloc_setup(Geo g, int rows, int cols, int lgN, unsigned char *__restri
 // have few butterflies in the first stage, so that the others' loads of
 // rho go out meanwhile.  For up to NOALLOC_FOLD row blocks (one per CU) that takes less
 // than the set-up launch it saves: allocation-free solve at 256^2 20.5 ->
-// 18.3 us, 512^2 22.2 -> 20.4, 1024x128 21.4 -> 20.2, 1024^2 36.8 -> 34.5; with more
+// 18.5 us, 512^2 22.2 -> 20.4, 1024x128 21.4 -> 19.7, 1024^2 36.9 -> 34.4; with more
 // the blocks' own tables cost more: 2048^2 (512 blocks) 64.8 -> 70.2.
 #define NOALLOC_FOLD 256
 template <int NT>
