@@ -1289,14 +1289,39 @@ launch_small(const SmallSolve &a, int P, size_t lds, hipStream_t stream)
 	return 0;
 }
 
-// Whether every plasma of the batch has the one-workgroup solve.
+// Plasmas of v values each up to which a batch of them is solved faster by a
+// workgroup of 1,024 threads per plasma than by the passes, whose blocks take
+// several small plasmas' share of the chip; 0: always.  Solve of P plasmas in us,
+// passes / workgroups:
+//   8x8     (32 values)    P = 1280 29.1 / 27.9   1536 32.8 / 33.0   4096 74.4 / 83.5
+//   16x8    (64)           1024 25.0 / 24.6       1152 28.9 / 29.9   2048 41.0 / 46.6
+//   16x16   (128)          768 22.3 / 20.6        896 25.7 / 26.5    4096 83.6 / 97.9
+//   32x16   (256)          1536 42.8 / 42.3       2048 53.8 / 55.4   4096 99.8 / 112.8
+//   32x32   (512)          1536 48.8 / 44.8       2048 58.6 / 60.7   4096 105.1 / 123.6
+//   64x32   (1024)         2304 81.7 / 77.5       3072 100.0 / 101.8 4096 128.6 / 134.4
+//   4x512   (1024)         2048 74.0 / 70.6       3072 98.8 / 104.0  4096 130.5 / 137.2
+//   64x64   (2048)         1024 62.4 / 45.1       2048 100.3 / 85.7  4096 202.6 / 177.6
+static int
+small_batch_limit(int64_t v)
+{
+	return v >= 2048 ? 0 : v >= 1024 ? 2304 : v >= 256 ? 1536 : v >= 128 ? 768 : v >= 64 ? 1024 : 1280;
+}
+
+// Whether the batch takes the one-workgroup solve: every plasma has it, and
+// their shares of the limits above come to at most 1.
 int
 cpic_solve_is_small(const cpic_dev *d)
 {
+	double share = 0.0;
 	for(int p = 0; p < d->P; p++)
+	{
+		const int limit = small_batch_limit(small_values(&d->hgeo[p]));
 		if(!small_ok(&d->hgeo[p]))
 			return 0;
-	return 1;
+		if(limit)
+			share += 1.0 / limit;
+	}
+	return share <= 1.0 + 1e-9;    // the rounding of the sum
 }
 
 static int
