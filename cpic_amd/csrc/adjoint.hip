@@ -442,10 +442,12 @@ static_assert(ADJ_CHUNK % REV_CHUNK == 0, "reverse blocks split the sort's chunk
 // Device memory the position history may take (16 B per particle and
 // iteration: 13.4 GB for 200 iterations of 4,194,304 particles), and at most
 // half of what is free.  The forward's push writes each iteration's positions
-// there instead of in place, at no extra traffic, and the reverse sweep reads
-// them instead of pushing every segment's particles again from a
-// checkpoint: 4,194,304 particles, 200 steps, forward and backward 78.4 -> 69.8 ms (11 ms of recompute);
-// the checkpoints (134 MB of copies each there) are not taken either.
+// there instead of in place.  It moves as many bytes, but 67 MB of them per
+// iteration to memory that the memory-side cache does not hold yet: push 53.5
+// -> 59.8 us, forward 15.9 -> 16.7 ms for 4,194,304 particles and 200 steps.  The
+// reverse sweep reads the positions instead of pushing every segment's
+// particles again from a checkpoint: 32.0 -> 21.2 ms.  The checkpoints (134 MB
+// of copies each there) are not taken.
 #define ADJ_POS_HISTORY_MAX ((int64_t) 32 << 30)
 template <bool PEND, int PPT>
 __global__ __launch_bounds__(CPIC_BLOCK)
@@ -580,8 +582,11 @@ void k_adj_rev_b(Geo g, AdjSpecies k, int64_t n, const uint8_t *__restrict__ sp,
 // run of ADJ_CHUNK positions the cells are taken round-robin: one particle of
 // every cell that still has one, per round, so that the 64 consecutive
 // particles of a wavefront lie in different cells and their deposit atomics
-// spread over the LDS banks (sort_by_cell_rr() in host_sort.h is the
-// sequential statement of it).  Counted, scanned and placed on the device;
+// spread over the LDS banks.  The particles of one cell come in the order in
+// which the counting reached them, another one in each forward: only sums
+// of deposits, whose order is open anyway, see it (sort_by_cell_rr() in host_sort.h
+// states the same order of cells sequentially, with the caller's order within
+// each).  Counted, scanned and placed on the device;
 // 4,194,304 particles at 256^2, a forward and a backward from host arrays:
 // 69.4 ms with the order made, applied and undone by 16 host threads, 48.2 ms so.
 

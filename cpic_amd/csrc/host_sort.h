@@ -1,8 +1,8 @@
-// Host side of the differentiable path's particle order, split over host
-// threads: a stable counting sort of the particles by cell with the cells of
-// each block chunk taken round-robin, and the gathers and scatters through
-// the resulting permutation.  Plain C++ (no HIP), so a host-only program can
-// check it against a sequential restatement.
+// Host threads for work on ranges, gathers through a permutation, and a
+// statement on the host of the differentiable run's particle order (a stable
+// counting sort by cell with the cells of each block chunk taken
+// round-robin), which the library makes on the device.  Plain C++ (no HIP), so a
+// host-only program can check it.
 #pragma once
 
 #include <stdint.h>
