@@ -525,6 +525,19 @@ cpic_dev_destroy(cpic_dev_t *d)
 
 // ---------------------------------------------------------- downloads ---
 
+// Queues the copy of one range and waits for the stream: the runtime stages what
+// the device does not reach.
+static int
+copy_plain(cpic_dev *d, int nr, const DlRange *r, bool up)
+{
+	hipError_t e = hipSuccess;
+	for(int k = 0; k < nr && e == hipSuccess; k++)
+		e = hipMemcpyAsync(r[k].dst, r[k].src, r[k].bytes,
+				up ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, d->stream);
+	hipError_t w = hipStreamSynchronize(d->stream);
+	return e == hipSuccess && w == hipSuccess ? 0 : CPIC_EHIP;
+}
+
 // Copies device ranges to ordinary host memory after the work queued on the
 // handle's stream, or (up) the other way.  Copying straight into pageable
 // memory runs at ~9 GB/s: the runtime's own staging is one thread's, and for a
@@ -536,7 +549,7 @@ cpic_dev_destroy(cpic_dev_t *d)
 // of 0.46 s sixteen of them took 7.1 s of CPU time.  Small copies run on the calling
 // thread: starting threads would cost more than they save.  Pinning costs ~0.1 ms per MB, once per
 // handle, so a handle that never copies more than 2 DL_CHUNK at once has
-// small buffers.
+// small buffers.  Where nothing can be pinned, the runtime stages the copies.
 #define COPY_POLL_US 500
 static int
 copy_ranges(cpic_dev *d, int nr, const DlRange *r, bool up)
@@ -556,7 +569,8 @@ copy_ranges(cpic_dev *d, int nr, const DlRange *r, bool up)
 		if(hipHostMalloc((void **) &d->pin, 2 * want, hipHostMallocDefault) != hipSuccess)
 		{
 			d->pin = NULL;
-			return CPIC_ENOMEM;
+			(void) hipGetLastError();
+			return copy_plain(d, nr, r, up);
 		}
 		d->pinchunk = want;
 	}
@@ -743,10 +757,17 @@ device_reaches(const void *p, size_t bytes)
 
 // Ranges whose host side the device reaches are one DMA each, the others go
 // through the bounce buffers: 128 MB into pinned memory 2.4 ms, with next to no CPU
-// time, where the bounce buffers' threads took 47-61 ms of it.
+// time, where the bounce buffers' threads took 47-61 ms of it.  One range alone, of
+// 16 to 512 KB, is as fast through the runtime's own staging, and needs no
+// buffers: field of 64 x 64 nodes read by a fresh handle 43 us through
+// buffers, 15 so, by one that has them 12.5 and 11.6; 256 x 256 64 and 35, 31.8 and 31.1.
+// Below, the runtime takes longer (2 KB 23 us, through buffers 16), above too (8 MB
+// 460, 430).
 static int
 copy_host(cpic_dev *d, int nr, const DlRange *r, bool up)
 {
+	if(nr == 1 && r[0].bytes >= DL_PLAIN_MIN && r[0].bytes <= DL_PLAIN_MAX)
+		return copy_plain(d, nr, r, up);
 	std::vector<DlRange> bounced;
 	int ret = 0;
 	bool direct = false;

@@ -44,6 +44,8 @@
 #define CPIC_MAX_KERNELS 24
 #define DL_CHUNK ((size_t) 4 << 20)      // bytes of a bounce buffer for host copies
 #define DL_CHUNK_SMALL ((size_t) 512 << 10)   // the same while no copy has exceeded 2 DL_CHUNK
+#define DL_PLAIN_MIN ((size_t) 16 << 10)      // single ranges of these sizes need no
+#define DL_PLAIN_MAX ((size_t) 512 << 10)     // bounce buffers (copy_host())
 #define DL_KEEP ((size_t) 256 << 20)     // largest download workspace a handle keeps
 
 // device error word bits
