@@ -1750,9 +1750,9 @@ void k_id_range(Geo g, Buckets bk, int par, Parts p, int s, DlInfo *__restrict__
 // `seen` (n bits, zero) particle i at position
 // i - info->lo, which the caller has found to be below n for all of them.
 // A particle's place in storage order is counted, not claimed, so that a state
-// gives the same rows in every call: the used slots of the rounds before,
-// of the wavefronts before in this round (one line of s_used, the lines
-// taking turns, so that one barrier per round does) and of the lanes before.
+// gives the same rows in every call: the used slots of the block's passes
+// before, of the wavefronts before in the same pass (one line of s_used, the
+// lines taking turns, so that one barrier per pass does) and of the lanes before.
 template <typename T, bool IDS, bool PE>
 __global__ __launch_bounds__(CPIC_BLOCK)
 void k_download(Geo g, Buckets bk, int par, Parts p, int s, const int64_t *__restrict__ off,
